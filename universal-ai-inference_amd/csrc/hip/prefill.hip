@@ -1562,6 +1562,8 @@ bool pf_supported(int type) {
 
 int64_t pf_mpad(int64_t m) { return (m + 63) / 64 * 64; }
 
+bool pf_row_supported(int64_t K) { return K * 4 <= lds_limit() - 2048; }
+
 hipError_t launch_pf_prep(float* x, int64_t ldx, int64_t M, const float* norm_w, float eps,
                           const PfAct& act, hipStream_t s, const float* part, int nsplit) {
   if (nsplit < 0 || (nsplit > 0 && !part)) return hipErrorInvalidValue;

@@ -319,7 +319,7 @@ struct PfQkvArgs {
 struct PfAttnArgs {
   const float* q;       // [M][ldq] post-RoPE
   int64_t ldq;
-  const void* kcache;   // f16 layer base [n_kv][max_seq][hd]
+  const void* kcache;   // layer base [n_kv][max_seq][hd], f16 (launch_pf_attn) or f32
   const void* vcache;
   int64_t max_seq;
   int n_heads, n_kv, hd;
@@ -347,6 +347,8 @@ bool pf_router_supported(int type);
 bool pf_supported(int type);
 bool pf_attn_supported(int head_dim, int n_heads, int n_kv);
 int64_t pf_mpad(int64_t m);
+// Whether launch_pf_prep (and the MoE routing) can stage a row of K values.
+bool pf_row_supported(int64_t K);
 // x [M][ldx] -> act. With nsplit > 0, x first becomes x + sum_z part[z][M][ldx]
 // (written back: x is the residual stream).
 hipError_t launch_pf_prep(float* x, int64_t ldx, int64_t M, const float* norm_w, float eps,
@@ -361,5 +363,7 @@ int pf_gemm_ksplit(const PfGemmArgs& a, int cus);
 int pf_gemm_group_rows(int type);
 hipError_t launch_pf_qkv(const PfQkvArgs& a, hipStream_t s);
 hipError_t launch_pf_attn(const PfAttnArgs& a, hipStream_t s);
+// The same over an f32 cache (prefill_attn_f32.hip).
+hipError_t launch_pf_attn_f32(const PfAttnArgs& a, hipStream_t s);
 
 }  // namespace uaii_hip

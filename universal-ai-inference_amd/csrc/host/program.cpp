@@ -118,7 +118,14 @@ void DecoderProgram::free_dynamic() {
 }
 
 Error DecoderProgram::charge(uint64_t& pool, uint64_t bytes) {
-  const uint64_t used = used_static_ + used_dyn_ + used_pf_;
+  uint64_t used = used_static_ + used_dyn_ + used_pf_;
+  // Prompt buffers that only speed a generate up (generate_rows) give way to
+  // what the session cannot do without.
+  if (opts_.budget_bytes != 0 && used + bytes > opts_.budget_bytes && !pf_ok_ && &pool != &used_pf_ && used_pf_ > 0) {
+    UAII_HIP(hipStreamSynchronize(stream_));
+    release_prefill_buffers();
+    used = used_static_ + used_dyn_;
+  }
   if (opts_.budget_bytes != 0 && used + bytes > opts_.budget_bytes)
     return Error::make(ErrorCode::InvalidArgument,
                        "memory budget exceeded: used=" + std::to_string(used) + " need=" +
@@ -334,10 +341,11 @@ Error DecoderProgram::build(const DecoderSpec& spec, const ProgramOptions& opts)
   int64_t want = opts_.max_context > 0 ? opts_.max_context : d.ctx_len;
   if (want > 0) UAII_TRY(ensure_capacity(want));
 
-  // the matrix-core prompt path: block formats it decodes, dense FFNs, f16 cache
-  pf_ok_ = opts_.kv_f16 && pf_attn_supported((int)d.head_dim, (int)d.n_heads, (int)d.n_kv_heads) &&
-           d.dim % 64 == 0 && d.q_dim % 64 == 0;
-  for (int64_t li = 0; pf_ok_ && li < d.n_layers; ++li) {
+  // the matrix-core prompt path: block formats it decodes, head sizes its
+  // attention takes
+  bool rows = pf_attn_supported((int)d.head_dim, (int)d.n_heads, (int)d.n_kv_heads) && d.dim % 64 == 0 &&
+              d.q_dim % 64 == 0;
+  for (int64_t li = 0; rows && li < d.n_layers; ++li) {
     const Layer& L = *layers_[(size_t)li];
     const LayerSpec& ls = d.layers[(size_t)li];
     std::vector<const DeviceWeight*> ws = {&L.wq, &L.wk, &L.wv, &L.wo};
@@ -347,15 +355,23 @@ Error DecoderProgram::build(const DecoderSpec& spec, const ProgramOptions& opts)
       ws.insert(ws.end(), {&L.gate_exps, &L.up_exps, &L.down_exps});
       if (L.shared) {
         ws.insert(ws.end(), {&L.gate_sh, &L.up_sh, &L.down_sh});
-        if (L.inter_sh % 64) pf_ok_ = false;
+        if (L.inter_sh % 64) rows = false;
       }
-      if (!pf_router_supported(L.gate_inp.view.type)) pf_ok_ = false;
+      if (!pf_router_supported(L.gate_inp.view.type)) rows = false;
     }
-    if (ls.ffn != LayerSpec::kNone && ls.inter % 64) pf_ok_ = false;
-    for (const DeviceWeight* w : ws) pf_ok_ = pf_ok_ && pf_supported(w->view.type);
+    if (ls.ffn != LayerSpec::kNone && ls.inter % 64) rows = false;
+    for (const DeviceWeight* w : ws) rows = rows && pf_supported(w->view.type);
   }
   if (const char* env = std::getenv("UAII_PREFILL")) {
-    if (std::string(env) == "0") pf_ok_ = false;
+    if (std::string(env) == "0") rows = false;
+  }
+  pf_ok_ = rows && opts_.kv_f16;
+  pf_rows_ = rows;
+  // a row longer than the prep stages runs in token steps (prefill() reports it)
+  if (!pf_ok_) {
+    pf_rows_ = pf_rows_ && pf_row_supported(d.dim) && pf_row_supported(d.q_dim);
+    for (const LayerSpec& ls : d.layers) pf_rows_ = pf_rows_ && pf_row_supported(ls.inter);
+    for (const auto& L : layers_) pf_rows_ = pf_rows_ && pf_row_supported(L->inter_sh);
   }
   // Q4_0 GEMMs take their high nibbles in place (PfAct::hi16) where every
   // consumer of a prep is one; UAII_PF_H16=0 keeps the shifted decode
@@ -382,12 +398,17 @@ Error DecoderProgram::build(const DecoderSpec& spec, const ProgramOptions& opts)
   return Error::success();
 }
 
-Error DecoderProgram::ensure_prefill_buffers(int64_t chunk) {
-  if (chunk <= pf_chunk_) return Error::success();
-  UAII_HIP(hipStreamSynchronize(stream_));
+void DecoderProgram::release_prefill_buffers() {
   for (void* p : pf_allocs_) (void)hipFree(p);
   pf_allocs_.clear();
   used_pf_ = 0;
+  pf_chunk_ = 0;
+}
+
+Error DecoderProgram::ensure_prefill_buffers(int64_t chunk) {
+  if (chunk <= pf_chunk_) return Error::success();
+  UAII_HIP(hipStreamSynchronize(stream_));
+  release_prefill_buffers();
   const DecoderSpec& d = spec_;
   int64_t inter = 1, inter_sh = 0;
   for (const LayerSpec& ls : d.layers) inter = std::max(inter, ls.inter);
@@ -644,24 +665,54 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
   return Error::success();
 }
 
+// Prompt tokens per pass: 1024 (on the 8B prompt 25.1k tok/s against 22.5k for
+// 512; 1536..4096 measured no better); UAII_PREFILL_CHUNK overrides.
+static int64_t prefill_chunk(int64_t n) {
+  int64_t target = 1024;
+  if (const char* env = std::getenv("UAII_PREFILL_CHUNK")) target = std::max<int64_t>(16, std::atoll(env));
+  return std::min(n, target);
+}
+
 Error DecoderProgram::prefill(int64_t n) {
   if (n <= 0) return Error::success();
   if (!pf_ok_) return Error::make(ErrorCode::NotImplemented, "prefill: model not covered by the matrix-core path");
+  return prefill_rows(n);
+}
+
+Error DecoderProgram::generate_rows(int64_t n, bool* done) {
+  *done = false;
+  if (n <= 0 || !pf_rows_) return Error::success();
+  if (pf_ok_) {
+    *done = true;
+    return prefill_rows(n);
+  }
+  // A few tokens are faster in steps: the layers' launches of the row path cost
+  // what 3 to 5 captured steps do (prompt of 4 / 6 tokens, f32 cache: 0.49 / 0.50
+  // against 0.49 / 0.69 ms on the 4-layer Q8_0 shape, 4.0 / 4.0 against 2.7 / 4.0
+  // ms on the 1B one).
+  if (n < 5) return Error::success();
+  // Such a session ran its prompt in token steps before this path took it, so
+  // it must not need the path's buffers: without the memory it still does.
+  if (!ensure_prefill_buffers(prefill_chunk(n)).ok()) {
+    (void)hipGetLastError();
+    release_prefill_buffers();
+    return Error::success();
+  }
+  *done = true;
+  return prefill_rows(n);
+}
+
+Error DecoderProgram::prefill_rows(int64_t n) {
   if (!kv_) return Error::make(ErrorCode::InvalidArgument, "KvCache not configured");
   const DecoderSpec& d = spec_;
   StepState st{};
   UAII_TRY(read_state(&st));
   const int64_t p0 = st.pos;
   if (p0 + n >= max_ctx_) return Error::make(ErrorCode::InvalidArgument, "prefill exceeds KV capacity");
-  // 1024-token chunks: on the 8B prompt 25.1k tok/s against 22.5k for 512 (the
-  // gate/up GEMM runs 8 % faster per token at M = 1024; 1536..4096 measured no
-  // better); UAII_PREFILL_CHUNK overrides
-  int64_t target = 1024;
-  if (const char* env = std::getenv("UAII_PREFILL_CHUNK")) target = std::max<int64_t>(16, std::atoll(env));
-  const int64_t chunk = std::min(n, target);
+  const int64_t chunk = prefill_chunk(n);
   UAII_TRY(ensure_prefill_buffers(chunk));
   hipStream_t s = stream_;
-  const size_t layer_kv = (size_t)d.kv_dim * (size_t)max_ctx_ * 2;
+  const size_t layer_kv = (size_t)d.kv_dim * (size_t)max_ctx_ * (opts_.kv_f16 ? 2 : 4);
   const int64_t ldqkv = d.q_dim + 2 * d.kv_dim;
   prof_used_ = 0;
   auto prep = [&](float* x, int64_t K, int64_t m, const float* norm_w, bool hi16 = false) -> Error {
@@ -738,7 +789,7 @@ Error DecoderProgram::prefill(int64_t n) {
       qa.qout = pf_q_;
       qa.kcache = kbase;
       qa.vcache = vbase;
-      qa.kv_f16 = 1;
+      qa.kv_f16 = opts_.kv_f16 ? 1 : 0;
       qa.max_seq = max_ctx_;
       UAII_TRY(timed("pf_qkv_rope", 4.0 * (double)m * (double)(ldqkv + d.q_dim + d.kv_dim), 0.0,
                      [&] { return launch_pf_qkv(qa, s); }));
@@ -758,7 +809,7 @@ Error DecoderProgram::prefill(int64_t n) {
       // causal (query, key) pairs x heads x (QK + PV) multiply-adds
       const double pairs = (double)m * (double)p + 0.5 * (double)m * (double)(m + 1);
       UAII_TRY(timed("pf_attention", 4.0 * pairs * (double)d.kv_dim, 4.0 * pairs * (double)d.q_dim, [&] {
-        return launch_pf_attn(at, s);
+        return opts_.kv_f16 ? launch_pf_attn(at, s) : launch_pf_attn_f32(at, s);
       }));
       UAII_TRY(prep(pf_attn_, d.q_dim, m, nullptr, h16(L.wo)));
       const DeviceWeight* wo[3] = {&L.wo, nullptr, nullptr};

@@ -96,6 +96,11 @@ class DecoderProgram {
   Error prefill(int64_t n);
   // Whether prefill() covers this model (weight formats, FFN kind, f16 KV cache).
   bool prefill_supported() const { return pf_ok_; }
+  // What generate() does with its prompt: the n tokens as prefill() takes them
+  // where the model's formats allow it, with either cache type. Not done (and
+  // nothing changed) where they do not, or where a session that prefill() does
+  // not cover has no memory for the path's buffers.
+  Error generate_rows(int64_t n, bool* done);
   // Overwrite the token fed at the current position.
   Error set_token(int64_t token);
   // Rewind to `pos` (ids and KV below it are kept; ids[pos] is fed next).
@@ -143,6 +148,8 @@ class DecoderProgram {
   Error timed(const char* name, double bytes, double flops, F&& launch);
   Error collect_timings();
   Error ensure_prefill_buffers(int64_t chunk);
+  void release_prefill_buffers();  // the stream must be idle
+  Error prefill_rows(int64_t n);
   Error pf_gemm(const DeviceWeight* w[3], const int64_t cols0[3], int nw, const DeviceWeight* w2,
                 int epi, int64_t m, float* y, int64_t ldy, int store_split = 1);
   int pf_store_split(const DeviceWeight* w[3], int nw, int64_t m, int64_t ldy);
@@ -209,7 +216,8 @@ class DecoderProgram {
   bool moe_ = false;
 
   // prefill: chunk buffers ([chunk][...] rows) and the prepared-activation scratch
-  bool pf_ok_ = false;
+  bool pf_ok_ = false;    // prefill(): the weights' formats and an f16 cache
+  bool pf_rows_ = false;  // generate_rows(): the weights' formats
   int64_t pf_chunk_ = 0, pf_kmax_ = 0;
   float *pf_x_ = nullptr, *pf_qkv_ = nullptr, *pf_q_ = nullptr, *pf_attn_ = nullptr,
         *pf_h_ = nullptr;

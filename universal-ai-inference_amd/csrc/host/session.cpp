@@ -122,8 +122,9 @@ Error Session::generate(const std::vector<int64_t>& prompt, int64_t max_new,
   // tokens but the last go through the matrix-core path as M-row products when
   // the model's formats allow it, and the last one runs the ordinary step with
   // the LM head. Otherwise one step per prompt token, logits only at the end.
-  if (n_prompt > 1 && p.prefill_supported()) {
-    UAII_TRY(p.prefill(n_prompt - 1));
+  bool rows_done = false;
+  if (n_prompt > 1) UAII_TRY(p.generate_rows(n_prompt - 1, &rows_done));
+  if (rows_done) {
     UAII_TRY(p.step(true));
   } else {
     for (int64_t i = 0; i < n_prompt; ++i) UAII_TRY(p.step(i == n_prompt - 1));
