@@ -45,6 +45,20 @@ enum : int {
   T_Q2_K = 10, T_Q3_K = 11, T_Q4_K = 12, T_Q5_K = 13, T_Q6_K = 14
 };
 
+// Compute units of the current device (queried once).
+inline int device_cus() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+      cus = v;
+    else
+      return 256;
+  }
+  return cus;
+}
+
 // Per-block LDS the current device allows (queried once; 64 KiB if unknown).
 inline int lds_limit() {
   static int lim = 0;

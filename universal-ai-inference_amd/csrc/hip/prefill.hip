@@ -9,97 +9,50 @@
 //   k_pf_prep   RMSNorm (optional) of each activation row, a power-of-two row
 //               scale 2^e, and the split x * 2^e = hi + lo into two f16 values
 //               (together ~22 significant bits), plus per-32 sums for formats
-//               whose blocks carry an offset.
-//   k_pf_gemm   C[M][N] = A . W^T with W read in its split GGUF layout: the
-//               weights of one (sub-)block decode in registers to their small
-//               integers, which f16 holds exactly; v_mfma_f32_16x16x32_f16
-//               (16x16x16 for 16-element sub-blocks) multiplies them with hi
-//               and with lo, and the block's scale (and offset times the row
-//               sum) is applied to the f32 partial. The only roundings are the
-//               f32 accumulations, so results match the f32 reference to
-//               ~1e-6 relative. Epilogues: store, residual add, SwiGLU, GELU.
+//               whose blocks carry a minimum.
+//   k_pf_mm     the products with the packed weights (prefill_gemm.hip).
 //   k_pf_qkv    Q/K/V bias, RoPE and the KV-cache append for M positions.
 //   k_pf_attn   causal attention of M queries over the f16 cache on MFMA:
 //               S^T = K . Q^T, online softmax, O^T += V^T . P^T, with q * scale
 //               and P split into f16 hi + lo against the exact f16 keys/values.
-//
-// Operand layout of the 16x16xK f16 MFMAs used here (CDNA3/CDNA4): lane l
-// supplies row (l % 16) of A and column (l % 16) of B with k-group (l / 16);
-// the f32 result D[4 * (l / 16) + r][l % 16] sits in element r of lane l. The
-// order of k inside a lane's group only has to agree between A and B: the
-// activation rows are stored with each aligned group of 4 values as
-// (k0, k2, k1, k3), the order in which the weight decode below produces them
-// from bytes 0 and 2, then 1 and 3, of a 32-bit word.
-#include <type_traits>
-
-#include "common.h"
-#include "uaii_hip_internal.h"
+#include "prefill.h"
 
 namespace uaii_hip {
 namespace {
 
-typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
-typedef float f4_t __attribute__((ext_vector_type(4)));
-
-__device__ inline h2_t as_h2(uint32_t u) { return __builtin_bit_cast(h2_t, u); }
-// (v & m) | c in one v_and_or_b32. Written out because gfx9's three-operand
-// encoding takes no literal constants, so the compiler splits the expression
-// into v_and + v_or; here the mask sits in a scalar register and the constant
-// in a vector register, both loop-invariant.
-__device__ inline uint32_t and_or(uint32_t v, uint32_t m, uint32_t c) {
-  uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(m), "v"(c));
-  return r;
-}
-// low nibbles of bytes 0 and 2 as f16 (1024 + q)
-__device__ inline uint32_t nib_pair(uint32_t v) { return and_or(v, 0x000F000Fu, 0x64006400u); }
-// The same with the mask in a vector register: 0x000F000F gives 1024 + q from
-// the low nibbles, 0x00F000F0 gives 1024 + 16 q from the high ones in place
-__device__ inline uint32_t and_or_v(uint32_t v, uint32_t m, uint32_t c) {
-  uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "v"(m), "v"(c));
-  return r;
-}
-// bytes 0 and 2 as f16 (1024 + b)
-__device__ inline uint32_t byte_pair(uint32_t v) { return and_or(v, 0x00FF00FFu, 0x64006400u); }
-
-__device__ inline h8_t cat8(h2_t a, h2_t b, h2_t c, h2_t d) {
-  return h8_t{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-}
-
-__device__ inline f4_t mfma32(h8_t a, h8_t b, f4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-__device__ inline float pow2f_i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
-
 // ---- activation prep ----------------------------------------------------------------
 
-// One block per row; rows >= M (tile padding) are written as zeros.
-__global__ void __launch_bounds__(256) k_pf_prep(float* __restrict__ x, int64_t ldx,
+// One block of NT threads per row; rows >= M (tile padding) are written as zeros.
+// Memory bound with many rows (13.4 us for 512 x 14336, 58 MB); with few it is a
+// chain of round trips, shorter with a row's loads spread over more threads.
+template <int NT>
+__global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t ldx,
                                                  int64_t M, const float* __restrict__ norm_w,
                                                  float eps, PfAct act, const float* __restrict__ part,
                                                  int nsplit) {
   extern __shared__ float row[];
-  __shared__ float red[4];
+  __shared__ float red[NT / 64];
   const int64_t t = blockIdx.x;
   const int tid = threadIdx.x;
   const int64_t K = act.K;
   const int nv = (int)(K / 4);
-  uint2* hi2 = reinterpret_cast<uint2*>(act.hi + t * K);
-  uint2* lo2 = reinterpret_cast<uint2*>(act.lo + t * K);
+  uint2* hi2 = reinterpret_cast<uint2*>(act.hi);
+  uint2* lo2 = reinterpret_cast<uint2*>(act.lo);
+  // float4 i of the row: quad i % 8 of 32-block i / 8, in the order 0, 4, 1, 5, ...
+  auto at = [&](int i) -> int64_t { return ((int64_t)(i >> 3) * act.mpad + t) * 8 + 2 * (i & 3) + ((i >> 2) & 1); };
   if (t >= M) {
-    for (int i = tid; i < nv; i += 256) { hi2[i] = make_uint2(0, 0); lo2[i] = make_uint2(0, 0); }
-    for (int64_t b = tid; b < K / 32; b += 256) act.sx[b * act.mpad + t] = 0.0f;
+    for (int i = tid; i < nv; i += NT) { hi2[at(i)] = make_uint2(0, 0); lo2[at(i)] = make_uint2(0, 0); }
+    if (act.sxp) {
+      for (int i = tid; i < nv / 8; i += NT)
+        reinterpret_cast<uint2*>(act.sxp)[((int64_t)(i >> 3) * act.mpad + t) * 8 + (i & 7)] = make_uint2(0, 0);
+    }
     if (tid == 0) act.rs[t] = 0.0f;
     return;
   }
   float4* r4 = reinterpret_cast<float4*>(row);
   float4* x4 = reinterpret_cast<float4*>(x + t * ldx);
   float ss = 0.0f, amax = 0.0f;
-  for (int i = tid; i < nv; i += 256) {
+  for (int i = tid; i < nv; i += NT) {
     float4 v = x4[i];
     if (nsplit > 0) {
       // residual add of a K-split GEMM's partials, in split order
@@ -120,11 +73,13 @@ __global__ void __launch_bounds__(256) k_pf_prep(float* __restrict__ x, int64_t 
     ss = wave_sum(ss);
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
-    const float tot = red[0] + red[1] + red[2] + red[3];
+    float tot = red[0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) tot += red[w];
     const float inv = 1.0f / sqrtf(tot / (float)K + eps);
     const float4* w4 = reinterpret_cast<const float4*>(norm_w);
     amax = 0.0f;
-    for (int i = tid; i < nv; i += 256) {
+    for (int i = tid; i < nv; i += NT) {
       float4 v = r4[i];
       const float4 w = w4[i];
       v.x = fmul_rn(fmul_rn(v.x, inv), w.x);
@@ -139,7 +94,8 @@ __global__ void __launch_bounds__(256) k_pf_prep(float* __restrict__ x, int64_t 
   amax = wave_max(amax);
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
-  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) amax = fmaxf(amax, red[w]);
   // scale so that max |x| * 2^e lies in [2^14, 2^15): hi keeps 11 bits of every
   // element near the top of the row and lo the next 11
   int e = 0;
@@ -149,774 +105,36 @@ __global__ void __launch_bounds__(256) k_pf_prep(float* __restrict__ x, int64_t 
   }
   const float s = pow2f_i(e);
   if (tid == 0) act.rs[t] = pow2f_i(-e);
-  for (int base = 0; base < nv; base += 256) {
+  for (int base = 0; base < nv; base += NT) {
     const int i = base + tid;
     float sum = 0.0f;
     if (i < nv) {
       const float4 v = r4[i];
       const float y0 = v.x * s, y1 = v.y * s, y2 = v.z * s, y3 = v.w * s;
-      // hi16 layout: elements 16..31 of the 32-block (float4 slots 4..7) times
-      // 1/16, exactly (a power of two), before the split
-      const float q = (act.hi16 && (i & 7) >= 4) ? 0.0625f : 1.0f;
-      const float z0 = y0 * q, z1 = y1 * q, z2 = y2 * q, z3 = y3 * q;
-      const _Float16 h0 = (_Float16)z0, h1 = (_Float16)z1, h2 = (_Float16)z2, h3 = (_Float16)z3;
-      const _Float16 l0 = (_Float16)(z0 - (float)h0), l1 = (_Float16)(z1 - (float)h1);
-      const _Float16 l2 = (_Float16)(z2 - (float)h2), l3 = (_Float16)(z3 - (float)h3);
+      const _Float16 h0 = (_Float16)y0, h1 = (_Float16)y1, h2 = (_Float16)y2, h3 = (_Float16)y3;
+      const _Float16 l0 = (_Float16)(y0 - (float)h0), l1 = (_Float16)(y1 - (float)h1);
+      const _Float16 l2 = (_Float16)(y2 - (float)h2), l3 = (_Float16)(y3 - (float)h3);
       // stored order (k0, k2, k1, k3)
-      hi2[i] = make_uint2(__builtin_bit_cast(uint32_t, h2_t{h0, h2}),
+      hi2[at(i)] = make_uint2(__builtin_bit_cast(uint32_t, h2_t{h0, h2}),
                           __builtin_bit_cast(uint32_t, h2_t{h1, h3}));
-      lo2[i] = make_uint2(__builtin_bit_cast(uint32_t, h2_t{l0, l2}),
+      lo2[at(i)] = make_uint2(__builtin_bit_cast(uint32_t, h2_t{l0, l2}),
                           __builtin_bit_cast(uint32_t, h2_t{l1, l3}));
       sum = (y0 + y1) + (y2 + y3);
     }
-    // 8 consecutive float4 = one 32-block (K % 32 == 0, so groups are whole)
-    sum += __shfl_xor(sum, 1, 64);
-    sum += __shfl_xor(sum, 2, 64);
-    sum += __shfl_xor(sum, 4, 64);
-    if (i < nv && (i & 7) == 0) act.sx[(int64_t)(i >> 3) * act.mpad + t] = sum;
-  }
-}
-
-// ---- weight fragments -----------------------------------------------------------------
-
-// A stage is two consecutive 32-blocks of k (kb = 2 st, 2 st + 1). PfRaw holds
-// the bytes of one weight row's stage that lane group g needs, loaded one stage
-// ahead of use; pf_decode() turns one block of it into the MFMA B operand (the
-// block's small integers) and its scale (and offset).
-template <int FMT>
-struct PfRaw;
-template <>
-struct PfRaw<T_Q4_0> {
-  uint2 q[2];   // qs bytes 8 (g & 1) .. +7 of each block
-  uint32_t d;   // the two f16 scales
-};
-template <>
-struct PfRaw<T_Q8_0> {
-  uint2 q[2];   // qs bytes 8 g .. +7 of each block
-  uint32_t d;
-};
-template <>
-struct PfRaw<T_Q4_K> {
-  uint2 q;      // qs bytes 8 g .. +7 of the pair: low nibbles block 0, high block 1
-  uint4 meta;   // d, dmin, scales[12] of the super-block
-};
-template <>
-struct PfRaw<T_Q6_K> {
-  uint2 ql[2];     // ql bytes 8 g .. +7 of blocks 0 and 1 (low or high nibbles by stage)
-  uint2 qh;        // qh bytes 8 g .. +7 (shared by both blocks)
-  uint32_t sc;     // the four int8 sub-block scales of the stage
-  uint32_t d;
-};
-
-template <int FMT>
-struct PfFrag {
-  h8_t b;         // the block's weight integers (Q6_K: the high part of sc (q - 32))
-  h8_t blo;       // Q6_K: the remainder of sc (q - 32) after b (0 or +-1)
-  float sc[1];
-  float off;
-};
-
-// Q6_K folds each 16-element sub-block's int8 scale into the MFMA operand:
-// sc (q - 32) is an integer of magnitude <= 4096, which the f16 pair (b, blo)
-// holds exactly, so a 32-element block (two sub-blocks) takes one 16x16x32 MFMA
-// per operand pair and only the super-block scale d remains for the f32 partial.
-template <int FMT>
-__device__ constexpr bool pf_split_b() {
-  return FMT == T_Q6_K;
-}
-template <int FMT>
-__device__ constexpr bool pf_offset() {
-  return FMT == T_Q4_K;
-}
-
-// The lane's row pointers into the split arrays, lane-group offsets folded in.
-struct PfRow {
-  const uint8_t* a;
-  const uint8_t* b;
-  const uint8_t* c;
-  const uint8_t* d;
-};
-
-template <int FMT>
-__device__ inline PfRow pf_row(const DevWeight& w, int64_t row, int g) {
-  PfRow p{};
-  p.a = w.a + row * w.a_row;
-  p.b = w.b + row * w.b_row;
-  if constexpr (FMT == T_Q4_0) {
-    p.a += 8 * (g & 1);
-  } else if constexpr (FMT == T_Q8_0 || FMT == T_Q4_K) {
-    p.a += 8 * g;
-  } else if constexpr (FMT == T_Q6_K) {
-    p.a += 8 * g;
-    p.b += 8 * g;
-    p.c = w.c + row * w.c_row;
-    p.d = w.d + row * w.d_row;
-  }
-  return p;
-}
-
-template <int FMT>
-__device__ inline void pf_load(const PfRow& p, int64_t st, PfRaw<FMT>& r) {
-  if constexpr (FMT == T_Q4_0) {
-    const uint8_t* q = p.a + st * 32;
-    r.q[0] = *reinterpret_cast<const uint2*>(q);
-    r.q[1] = *reinterpret_cast<const uint2*>(q + 16);
-    r.d = *reinterpret_cast<const uint32_t*>(p.b + st * 4);
-  } else if constexpr (FMT == T_Q8_0) {
-    const uint8_t* q = p.a + st * 64;
-    r.q[0] = *reinterpret_cast<const uint2*>(q);
-    r.q[1] = *reinterpret_cast<const uint2*>(q + 32);
-    r.d = *reinterpret_cast<const uint32_t*>(p.b + st * 4);
-  } else if constexpr (FMT == T_Q4_K) {
-    r.q = *reinterpret_cast<const uint2*>(p.a + st * 32);
-    r.meta = *reinterpret_cast<const uint4*>(p.b + (st >> 2) * 16);
-  } else if constexpr (FMT == T_Q6_K) {
-    // super-block st / 4, half (st % 4) / 2, elements 64 (st % 2) .. +63 of the half
-    const uint8_t* ql = p.a + (st >> 1) * 64;
-    r.ql[0] = *reinterpret_cast<const uint2*>(ql);
-    r.ql[1] = *reinterpret_cast<const uint2*>(ql + 32);
-    r.qh = *reinterpret_cast<const uint2*>(p.b + (st >> 1) * 32);
-    r.sc = *reinterpret_cast<const uint32_t*>(p.c + st * 4);
-    r.d = ld_u16(p.d + (st >> 2) * 2);
-  }
-}
-
-// Block s (0 or 1) of stage st for lane group g. H16 (Q4_0, PfAct::hi16
-// activations): lane groups 2 and 3, which hold elements 16..31, decode their
-// high nibbles in place as 16 (q - 8), exact in f16, and the activations of
-// those elements carry the factor 1/16; this saves the per-lane shift.
-template <int FMT, bool H16 = false>
-__device__ inline void pf_decode(const PfRaw<FMT>& r, int64_t st, int s, int g, PfFrag<FMT>& f) {
-  if constexpr (FMT == T_Q4_0 && H16) {
-    const bool up = g >= 2;
-    const uint32_t m = up ? 0x00F000F0u : 0x000F000Fu;
-    const _Float16 bv = up ? (_Float16)1152.0f : (_Float16)1032.0f;  // 1024 + 16 * 8 : 1024 + 8
-    const h2_t bias = {bv, bv};
-    const uint32_t c = 0x64006400u;
-    const uint32_t v0 = r.q[s].x, v1 = r.q[s].y;
-    f.b = cat8(as_h2(and_or_v(v0, m, c)) - bias, as_h2(and_or_v(v0 >> 8, m, c)) - bias,
-               as_h2(and_or_v(v1, m, c)) - bias, as_h2(and_or_v(v1 >> 8, m, c)) - bias);
-    f.sc[0] = h2f((uint16_t)(r.d >> (16 * s)));
-  } else if constexpr (FMT == T_Q4_0) {
-    const int sh = (g >> 1) * 4;
-    const uint32_t v0 = r.q[s].x >> sh, v1 = r.q[s].y >> sh;
-    const h2_t bias = {(_Float16)1032.0f, (_Float16)1032.0f};
-    f.b = cat8(as_h2(nib_pair(v0)) - bias, as_h2(nib_pair(v0 >> 8)) - bias,
-               as_h2(nib_pair(v1)) - bias, as_h2(nib_pair(v1 >> 8)) - bias);
-    f.sc[0] = h2f((uint16_t)(r.d >> (16 * s)));
-  } else if constexpr (FMT == T_Q8_0) {
-    const uint32_t v0 = r.q[s].x ^ 0x80808080u, v1 = r.q[s].y ^ 0x80808080u;
-    const h2_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-    f.b = cat8(as_h2(byte_pair(v0)) - bias, as_h2(byte_pair(v0 >> 8)) - bias,
-               as_h2(byte_pair(v1)) - bias, as_h2(byte_pair(v1 >> 8)) - bias);
-    f.sc[0] = h2f((uint16_t)(r.d >> (16 * s)));
-  } else if constexpr (FMT == T_Q4_K) {
-    const int j = 2 * (int)(st & 3) + s;  // sub-block of the super-block
-    const uint32_t v0 = r.q.x >> (4 * s), v1 = r.q.y >> (4 * s);
-    const h2_t bias = {(_Float16)1024.0f, (_Float16)1024.0f};
-    f.b = cat8(as_h2(nib_pair(v0)) - bias, as_h2(nib_pair(v0 >> 8)) - bias,
-               as_h2(nib_pair(v1)) - bias, as_h2(nib_pair(v1 >> 8)) - bias);
-    // 6-bit (scale, min) pair j of the 12-byte field (gguf_dequant.cpp:107-115):
-    // bytes j & 3 of the three words hold s[j & 3], s[4 + (j & 3)], s[8 + (j & 3)]
-    const int bsh = 8 * (j & 3);
-    const int by = (int)((r.meta.y >> bsh) & 0xff), bz = (int)((r.meta.z >> bsh) & 0xff);
-    const int bw = (int)((r.meta.w >> bsh) & 0xff);
-    int sc, mn;
-    if (j < 4) {
-      sc = by & 63;
-      mn = bz & 63;
-    } else {
-      sc = (bw & 15) | ((by >> 6) << 4);
-      mn = (bw >> 4) | ((bz >> 6) << 4);
-    }
-    const float d = h2f((uint16_t)(r.meta.x & 0xffff)), dmin = h2f((uint16_t)(r.meta.x >> 16));
-    f.sc[0] = fmul_rn(d, (float)sc);
-    f.off = fmul_rn(dmin, (float)mn);
-  } else if constexpr (FMT == T_Q6_K) {
-    // element e = 64 (st % 2) + 32 s + 8 g + i of the half: ql byte e % 64 (high
-    // nibble when e >= 64), qh byte e % 32 at bit 2 (e / 32), sub-block e / 16 of
-    // the stage, i.e. 2 s + g / 2. b = RN(sc (q - 32)) and blo = sc (q - 32) - b
-    // by one fused multiply-add, exact: the integer is at most 4096 in magnitude
-    const int nib = (int)(st & 1) * 4;
-    const int qsh = 4 * (int)(st & 1) + 2 * s;
-    const h2_t bias = {(_Float16)1056.0f, (_Float16)1056.0f};
-    const _Float16 scv = (_Float16)(float)(int8_t)((r.sc >> (8 * (2 * s + (g >> 1)))) & 0xff);
-    const h2_t sc2 = {scv, scv};
-    const uint32_t w[2] = {r.ql[s].x, r.ql[s].y}, hq[2] = {r.qh.x, r.qh.y};
-    h2_t hi[4], lo[4];
+    if (act.sxp) {
+      // 8 consecutive float4 = one 32-block, 64 a super-block (K % 256 == 0)
+      sum += __shfl_xor(sum, 1, 64);
+      sum += __shfl_xor(sum, 2, 64);
+      sum += __shfl_xor(sum, 4, 64);
+      if (i < nv && (i & 7) == 0) {
+        _Float16* d = reinterpret_cast<_Float16*>(act.sxp) + ((int64_t)(i >> 6) * act.mpad + t) * 32 + ((i >> 3) & 7);
+        float v = sum * 0.03125f;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const uint32_t q6 = ((w[t] >> nib) & 0x0F0F0F0Fu) | (((hq[t] >> qsh) & 0x03030303u) << 4);
-      const h2_t p0 = as_h2(byte_pair(q6)) - bias, p1 = as_h2(byte_pair(q6 >> 8)) - bias;
-      hi[2 * t] = p0 * sc2;
-      lo[2 * t] = __builtin_elementwise_fma(p0, sc2, -hi[2 * t]);
-      hi[2 * t + 1] = p1 * sc2;
-      lo[2 * t + 1] = __builtin_elementwise_fma(p1, sc2, -hi[2 * t + 1]);
-    }
-    f.b = cat8(hi[0], hi[1], hi[2], hi[3]);
-    f.blo = cat8(lo[0], lo[1], lo[2], lo[3]);
-    f.sc[0] = h2f((uint16_t)r.d);
-  }
-}
-
-// ---- GEMM -------------------------------------------------------------------------------
-
-#ifndef UAII_PF_DMA
-#define UAII_PF_DMA 1  // Q4_0 / Q8_0 through the direct-to-LDS kernel
-#endif
-#ifndef UAII_PF_TILE
-#define UAII_PF_TILE 0  // wave tile: 0 chosen per launch, 2 64x32, 3 32x32
-#endif
-constexpr int PF_WAVES = 4;   // waves per block, side by side along N
-#ifndef UAII_PF_KTILE
-#define UAII_PF_KTILE 1  // Q4_K takes the 64 x 32 wave tile too (0: always 32 x 32)
-#endif
-#ifndef UAII_PF_ROW
-#define UAII_PF_ROW 40
-#endif
-#ifndef UAII_PF_KS_BPC
-// K split target: four-wave block equivalents per CU. 4 (two 8-wave blocks per
-// CU) measured 26.2k against 25.5k tok/s for 2 on the 8B prompt (down, O and
-// QKV 3-12 % faster, the partial fold in the next prep 1.4 ms slower); 8 25.2k
-#define UAII_PF_KS_BPC 4
-#endif
-#ifndef UAII_PF_K6TILE
-// Q6_K takes the 64 x 32 wave tile where the grid allows (0: always 32 x 32):
-// 1B down 14.3 -> 11.3 ms per prompt with the former 16x16x16 decode
-#define UAII_PF_K6TILE 1
-#endif
-#ifndef UAII_PF_DW
-#define UAII_PF_DW 8  // waves per block of the direct-to-LDS kernel (4 or 8)
-#endif
-#ifndef UAII_PF_XCD
-#define UAII_PF_XCD 1  // XCD-aware block order in the direct-to-LDS kernel
-#endif
-constexpr int PF_ROW = UAII_PF_ROW;  // halfs per staged 32-k row (32 + 8 pad)
-
-// LDS: [buffer 2][block 2][hi/lo 2][BM rows][PF_ROW halfs]
-template <int MT>
-constexpr int pf_lds_halfs() { return 2 * 2 * 2 * 16 * MT * PF_ROW; }
-
-// Output rows [m0, mend) of this grid row and the first weight row of its
-// expert (0 without grouping).
-struct PfRange {
-  int64_t m0, mend, mfirst, wrow0;
-};
-__device__ inline PfRange pf_range(const PfGemmArgs& a, int bm, int64_t seg_rows, int gy = -1) {
-  if (gy < 0) gy = blockIdx.y;
-  PfRange r;
-  if (a.gtab) {
-    const int32_t* e = a.gtab + 3 * gy;
-    r.wrow0 = (int64_t)e[0] * seg_rows;
-    r.m0 = e[1];
-    r.mend = e[2];
-    r.mfirst = r.m0;
-  } else {
-    r.wrow0 = 0;
-    r.m0 = (int64_t)gy * bm;
-    r.mend = a.M;
-    r.mfirst = 0;
-  }
-  return r;
-}
-// Activation row of output row t. Rows past the range read its first row (the
-// map's first entry without grouping); their results are dropped. Unmapped,
-// ungrouped rows below mpad are read as they are.
-__device__ inline int64_t pf_arow(const PfGemmArgs& a, const PfRange& r, int64_t t) {
-  if (!a.arow && !a.gtab) return t;
-  const int64_t tc = t < r.mend ? t : r.mfirst;
-  return a.arow ? (int64_t)a.arow[tc] : tc;
-}
-
-// Block tile: 16 MT activation rows x PF_WAVES * 16 NT weight rows (for SwiGLU
-// each wave's NT subtiles are NT / 2 gate and NT / 2 up subtiles of the same
-// rows). K advances one stage (64) at a time; activations are staged in LDS
-// (double-buffered), each lane loads its weight bytes one stage ahead.
-template <int FMT, int EPI, int MT, int NT>
-__global__ void __launch_bounds__(PF_WAVES * 64, 2) k_pf_gemm(PfGemmArgs a) {
-  constexpr int BM = 16 * MT;
-  constexpr bool OFF = pf_offset<FMT>();
-  constexpr int NQ = (EPI == EPI_SWIGLU) ? NT / 2 : NT;  // distinct row subtiles
-  __shared__ _Float16 lds[pf_lds_halfs<MT>()];
-
-  // segment of this column tile
-  const int tile = blockIdx.x;
-  int si = 0;
-  for (int k = 1; k < a.nseg; ++k) if (tile >= a.seg[k].tile0) si = k;
-  const PfSeg& seg = a.seg[si];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int col = lane & 15, g = lane >> 4;
-  const int64_t n0 = ((int64_t)(tile - seg.tile0) * PF_WAVES + wave) * (16 * NQ);
-  const PfRange mr = pf_range(a, BM, seg.rows);
-  const int64_t m0 = mr.m0;
-  const int64_t K = a.K, nst = K / 64 / a.ksplit;  // stages of this block's K range
-  const int64_t sbase = (int64_t)blockIdx.z * nst;  // its first stage
-
-  // weight rows of this lane per subtile (clamped: rows past the end are loaded, not stored)
-  PfRow prow[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int64_t r = n0 + 16 * (j % NQ) + col;
-    const DevWeight& w = (EPI == EPI_SWIGLU && j >= NQ) ? seg.w2 : seg.w;
-    prow[j] = pf_row<FMT>(w, mr.wrow0 + (r < seg.rows ? r : seg.rows - 1), g);
-  }
-
-  f4_t acc[MT][NT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-  auto arow_of = [&](int64_t t) __attribute__((always_inline)) -> int64_t { return pf_arow(a, mr, t); };
-  // activation stage: BM rows x 2 blocks x (hi, lo) x 4 pieces of 16 B
-  constexpr int PIECES = BM * 2 * 2 * 4;
-  constexpr int PPT = PIECES / (PF_WAVES * 64);
-  static_assert(PIECES % (PF_WAVES * 64) == 0, "stage pieces per thread");
-  // activation pieces one stage ahead (stored to the other LDS buffer after the
-  // compute), weight bytes two stages ahead in a ring of 3; ring indices are
-  // compile-time constants
-  uint4 stg[PPT];
-  PfRaw<FMT> raw[3][NT];
-  // this thread's activation pieces at stage 0 of the block's K range (a stage
-  // adds 64 halfs); row offsets and the row map are read once, not per stage
-  const __half* abase[PPT];
-#pragma unroll
-  for (int u = 0; u < PPT; ++u) {
-    const int c = threadIdx.x + u * PF_WAVES * 64;
-    const int q = c & 3, r = (c >> 2) % BM, kbh = (c >> 2) / BM;  // kbh = block * 2 + hi/lo
-    abase[u] = ((kbh & 1) ? a.alo : a.ahi) + arow_of(m0 + r) * K + (2 * sbase + (kbh >> 1)) * 32 + q * 8;
-  }
-  // Q4_K: the activation block sums of the stage's two blocks, staged beside the
-  // activations (threads < 2 BM, one value each) instead of read from memory
-  // inside the compute, where the wait for them would also wait for every load
-  // in flight
-  __shared__ float sxs[OFF ? 2 * 2 * BM : 1];
-  float stg_sx = 0.0f;
-  const float* sxbase = nullptr;
-  if constexpr (OFF) {
-    const int t = threadIdx.x < 2 * BM ? threadIdx.x : 0;
-    sxbase = a.sx + (2 * sbase + t / BM) * a.sx_ld + arow_of(m0 + t % BM);
-  }
-  auto load_stage = [&](uint4 (&dst)[PPT], int64_t st) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < PPT; ++u) {
-      // element-wise: a whole-struct copy here is turned into a memcpy into a
-      // stack array (scratch memory)
-      const uint4 v = *reinterpret_cast<const uint4*>(abase[u] + st * 64);
-      dst[u].x = v.x;
-      dst[u].y = v.y;
-      dst[u].z = v.z;
-      dst[u].w = v.w;
-    }
-    if constexpr (OFF) stg_sx = sxbase[st * 2 * a.sx_ld];
-  };
-  auto store_stage = [&](const uint4 (&src)[PPT], int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < PPT; ++u) {
-      const int c = threadIdx.x + u * PF_WAVES * 64;
-      const int q = c & 3, r = (c >> 2) % BM, kbh = (c >> 2) / BM;
-      _Float16* dst = lds + (((buf * 4) + kbh) * BM + r) * PF_ROW + q * 8;
-      *reinterpret_cast<uint4*>(dst) = src[u];
-    }
-    if constexpr (OFF) {
-      if (threadIdx.x < 2 * BM) sxs[buf * 2 * BM + threadIdx.x] = stg_sx;
-    }
-  };
-  auto load_w = [&](PfRaw<FMT>(&dst)[NT], int64_t st) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < NT; ++j) pf_load<FMT>(prow[j], sbase + st, dst[j]);
-  };
-  // LDS writes done, then the block barrier. No memory fence: a fence would also
-  // wait for the weight and activation loads in flight for later stages.
-  auto lds_barrier = []() __attribute__((always_inline)) {
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0); vmcnt, expcnt untouched
-    __builtin_amdgcn_s_barrier();
-  };
-  auto compute = [&](const PfRaw<FMT>(&rw)[NT], int64_t stl, int buf) __attribute__((always_inline)) {
-    const int64_t st = sbase + stl;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      PfFrag<FMT> fr[NT];
-#pragma unroll
-      for (int j = 0; j < NT; ++j) pf_decode<FMT>(rw[j], st, s, g, fr[j]);
-      const _Float16* base = lds + ((buf * 2 + s) * 2) * BM * PF_ROW;
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const _Float16* ph = base + (16 * i + col) * PF_ROW;
-        const _Float16* pl = ph + BM * PF_ROW;
-        f4_t sxv = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        if constexpr (OFF) {
-          const float4 s4 = *reinterpret_cast<const float4*>(sxs + (buf * 2 + s) * BM + 16 * i + 4 * g);
-          sxv = f4_t{s4.x, s4.y, s4.z, s4.w};
+        for (int p = 0; p < 3; ++p) {
+          d[8 * p] = (_Float16)v;
+          v -= (float)d[8 * p];
         }
-        const h8_t ahi = *reinterpret_cast<const h8_t*>(ph + 8 * g);
-        const h8_t alo = *reinterpret_cast<const h8_t*>(pl + 8 * g);
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          f4_t p = mfma32(ahi, fr[j].b, f4_t{0.0f, 0.0f, 0.0f, 0.0f});
-          p = mfma32(alo, fr[j].b, p);
-          if constexpr (pf_split_b<FMT>()) p = mfma32(ahi, fr[j].blo, p);  // (hi, lo) x lo: ~2^-21
-          acc[i][j] += fr[j].sc[0] * p;
-          if constexpr (OFF) acc[i][j] -= fr[j].off * sxv;
-        }
-      }
-    }
-  };
-  // one stage: prefetch activations of st + 1 and weights of st + 2, compute
-  // stage st, move stage st + 1 into the other LDS buffer
-  auto step = [&](auto ws, int64_t st) __attribute__((always_inline)) {
-    constexpr int W = decltype(ws)::value;
-    if (st + 1 < nst) load_stage(stg, st + 1);
-    if (st + 2 < nst) load_w(raw[(W + 2) % 3], st + 2);
-    compute(raw[W], st, (int)(st & 1));
-    if (st + 1 < nst) store_stage(stg, (int)((st + 1) & 1));
-    lds_barrier();
-  };
-
-  load_w(raw[0], 0);
-  if (nst > 1) load_w(raw[1], 1);
-  load_stage(stg, 0);
-  store_stage(stg, 0);
-  lds_barrier();
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  for (int64_t st = 0; st < nst; st += 3) {
-    step(I0{}, st);
-    if (st + 1 >= nst) break;
-    step(I1{}, st + 1);
-    if (st + 2 >= nst) break;
-    step(I2{}, st + 2);
-  }
-
-  // epilogue: lane holds rows m0 + 16i + 4g + r of column n0 + 16j + col
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t t = m0 + 16 * i + 4 * g + r;
-      if (t >= mr.mend) continue;
-      const float rs = a.rs[pf_arow(a, mr, t)];
-      float* yrow = a.y + t * a.ldy + seg.col0;
-#pragma unroll
-      for (int j = 0; j < NQ; ++j) {
-        const int64_t n = n0 + 16 * j + col;
-        if (n >= seg.rows) continue;
-        const float v = acc[i][j][r] * rs;
-        if constexpr (EPI == EPI_STORE) {
-          if (a.ksplit > 1) a.part[((int64_t)blockIdx.z * a.M + t) * a.ldy + seg.col0 + n] = v;
-          else yrow[n] = v;
-        } else if constexpr (EPI == EPI_ADD) {
-          if (a.ksplit > 1) a.part[((int64_t)blockIdx.z * a.M + t) * a.ldy + seg.col0 + n] = v;
-          else yrow[n] = yrow[n] + v;
-        } else if constexpr (EPI == EPI_SWIGLU) {
-          const float u = acc[i][j + NQ][r] * rs;
-          const float act = v / (1.0f + expf(-v));  // silu (elementwise.cpp:73-84)
-          yrow[n] = act * u;
-        } else if constexpr (EPI == EPI_GELU) {
-          const float inner = 0.7978845608f * (v + 0.044715f * v * v * v);
-          yrow[n] = 0.5f * v * (1.0f + tanhf(inner));
-        }
-      }
-    }
-  }
-}
-
-// ---- GEMM with direct-to-LDS loads (Q4_0, Q8_0) -----------------------------------------
-//
-// Same tile math as k_pf_gemm, but activations and weight bytes travel global ->
-// LDS with global_load_lds_dwordx4 / _dword (lane i of an instruction writes the
-// 16 (4) bytes at M0 + 16 i (4 i)), so no registers hold data in flight and a
-// ring of three LDS stages keeps two stages of loads outstanding. The loads are
-// issued from inline assembly and their completion is waited for with explicit
-// vmcnt counts: the compiler would otherwise wait for every outstanding LDS
-// load before each LDS read. Both operands stay row-major in LDS (the lanes
-// of one DMA instruction that share a row fetch its contiguous bytes), with
-// the 16-byte pieces of each row XOR-permuted so that the fragment reads are
-// free of bank conflicts on gfx950: activation piece p of row r sits in slot
-// p ^ ((r >> 1) & 3); weight part p of row r (32- or 64-byte rows) in slot
-// p ^ ((r >> 3) & 1) for Q4_0, p ^ ((r >> 2) & 3) for Q8_0. Measured with
-// SQ_LDS_BANK_CONFLICT: unpermuted rows cost 4 conflict cycles per 16-byte
-// activation read and 2 (Q4_0) or 6 (Q8_0) per 8-byte weight read, as does
-// the permutation p ^ (((r >> 1) ^ (r >> 3)) & 3) for the activations.
-//
-// The LDS address goes to the asm as an M0 operand ("{m0}"), so the compiler
-// writes M0 itself and knows it holds that value; the s_nop gives the one wait
-// state an LDS DMA needs after an M0 write.
-
-__device__ inline void dma16(const void* g, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(g) : "memory");
-}
-__device__ inline void dma4(const void* g, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dword %1, off" ::"{m0}"(lds), "v"(g) : "memory");
-}
-// The same 16-byte copy from a wave-uniform base (scalar registers) plus the
-// lane's 32-bit byte offset: no per-lane 64-bit address arithmetic per stage.
-__device__ inline void dma16s(const void* sbase, uint32_t voff, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(voff), "s"(sbase)
-               : "memory");
-}
-// A pointer the wave holds in common, made visibly uniform so that it lives in
-// scalar registers.
-__device__ inline const uint8_t* uniform_ptr(const void* p) {
-  const uint64_t u = (uint64_t)(uintptr_t)p;
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
-  return reinterpret_cast<const uint8_t*>((uintptr_t)(((uint64_t)hi << 32) | lo));
-}
-__device__ inline uint32_t lds_addr(const void* p) {
-  return __builtin_amdgcn_readfirstlane(
-      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
-}
-__device__ inline int pf_swz(int r) { return (r >> 1) & 3; }
-template <int FMT>
-__device__ inline int pf_wswz(int r) { return FMT == T_Q4_0 ? (r >> 3) & 1 : (r >> 2) & 3; }
-
-template <int FMT>
-constexpr int dma_qbytes() { return FMT == T_Q8_0 ? 64 : 32; }  // payload bytes per row per stage
-template <int MT>
-constexpr int dma_a_bytes() { return 2 * 2 * 16 * MT * 64; }      // [block][hi/lo][row][64 B]
-// per wave: the payload of its 16 NT rows, then a 256-byte scale area (a dword per row)
-template <int FMT, int NT>
-constexpr int dma_wave_w_bytes() { return 16 * NT * dma_qbytes<FMT>() + 256; }
-// Waves per block of the direct-to-LDS kernel, side by side along N: 8, so
-// that with two blocks per CU each SIMD holds four waves.
-constexpr int PF_DW = UAII_PF_DW;
-template <int FMT, int MT, int NT>
-constexpr int dma_stage_bytes() { return dma_a_bytes<MT>() + PF_DW * dma_wave_w_bytes<FMT, NT>(); }
-// Activation DMA instructions per wave and stage: the 4 MT (block, hi/lo,
-// subtile) copies spread over the waves
-template <int MT>
-constexpr int dma_a_per_wave() { return 4 * MT / PF_DW; }
-// DMA instructions each wave issues per stage (the vmcnt unit)
-template <int FMT, int MT, int NT>
-constexpr int dma_per_stage() { return dma_a_per_wave<MT>() + 16 * NT * dma_qbytes<FMT>() / 1024 + 1; }
-// Weight subtiles per wave: 2 (32 rows). 64-row waves (4) spilled registers at
-// the 64 x 64 wave tile.
-template <int FMT>
-constexpr int dma_nt() { return 2; }
-
-template <int FMT, int EPI, int MT, int NT, bool H16>
-__global__ void __launch_bounds__(PF_DW * 64, 2) k_pf_gemm_dma(PfGemmArgs a) {
-  static_assert(NT == 2 || NT == 4, "weight subtiles per wave");
-  static_assert((4 * MT) % PF_DW == 0, "activation copies per wave");
-  constexpr int NA = dma_a_per_wave<MT>();
-  constexpr int BM = 16 * MT;
-  constexpr int NQ = (EPI == EPI_SWIGLU) ? NT / 2 : NT;
-  constexpr int NR = 16 * NT;  // weight rows per wave
-  constexpr int QB = dma_qbytes<FMT>();
-  constexpr int WB = dma_wave_w_bytes<FMT, NT>();
-  constexpr int SB = dma_stage_bytes<FMT, MT, NT>();
-  constexpr int ND = dma_per_stage<FMT, MT, NT>();
-  static_assert(ND <= 15, "vmcnt immediate");
-  __shared__ __attribute__((aligned(16))) uint8_t lds[3 * SB];
-
-  // Grid position. Blocks go to the XCDs round-robin in dispatch order; with
-  // the column-tile count a multiple of 8, XCD x takes the column tiles
-  // 8 c + x, and within an XCD the blocks are renumbered row tile fastest, so
-  // that the blocks resident on one XCD share their weight columns in its L2.
-  int tile = blockIdx.x, gy = blockIdx.y;
-#if UAII_PF_XCD
-  if ((gridDim.x & 7) == 0) {
-    const int id = blockIdx.y * gridDim.x + blockIdx.x;
-    const int loc = id >> 3;
-    gy = loc % gridDim.y;
-    tile = (loc / gridDim.y) * 8 + (id & 7);
-  }
-#endif
-  int si = 0;
-  for (int k = 1; k < a.nseg; ++k) if (tile >= a.seg[k].tile0) si = k;
-  const PfSeg& seg = a.seg[si];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int col = lane & 15, g = lane >> 4;
-  const int64_t n0 = ((int64_t)(tile - seg.tile0) * PF_DW + wave) * (16 * NQ);
-  const PfRange mr = pf_range(a, BM, seg.rows, gy);
-  const int64_t m0 = mr.m0;
-  const int64_t K = a.K;
-  const int nst = (int)(K / 64 / a.ksplit);         // stages of this block's K range
-  const int64_t sbase = (int64_t)blockIdx.z * nst;  // its first stage
-
-  // this lane's DMA sources. Activations: wave w copies (block (w >> 1) & 1,
-  // hi/lo w & 1) of the row subtiles NA (w >> 2) .. NA (w >> 2) + NA - 1;
-  // instruction u covers rows 16 u' .. 16 u' + 15 of its subtile u', lane ->
-  // (row, slot).
-  const int arow_l = lane >> 2, aslot = lane & 3;
-  const __half* asrc = (wave & 1) ? a.alo : a.ahi;
-  const int ablk = (wave >> 1) & 1;
-  const int asub0 = NA * (wave >> 2);
-  // the lane's byte offset of its row's piece (stage independent; the launch
-  // checks that the activation array spans under 2^31 bytes) and the wave's
-  // scalar base, to which stage st adds 128 st bytes (64 k of f16)
-  uint32_t aoff[NA];
-#pragma unroll
-  for (int u = 0; u < NA; ++u) {
-    const int r = 16 * (asub0 + u) + arow_l;
-    const int piece = aslot ^ pf_swz(r);
-    aoff[u] = (uint32_t)(pf_arow(a, mr, m0 + r) * K * 2) + (uint32_t)(ablk * 64 + piece * 16);
-  }
-  const uint8_t* abase = uniform_ptr(asrc);
-  // Weights: the wave's 32 rows (subtile j = row / 16; SwiGLU: j = 1 is the up
-  // tensor); a row's stage payload is WP 16-byte parts, and LDS slot
-  // q = 64 u + lane of the payload is slot q % WP of row q / WP. One dword per
-  // row of scales.
-  constexpr int WP = QB / 16;
-  constexpr int NWQ = NR * QB / 1024;  // payload DMA instructions per stage
-  const uint8_t* wsrc_q[NWQ];
-#pragma unroll
-  for (int u = 0; u < NWQ; ++u) {
-    const int q = lane + 64 * u;
-    const int rl = q / WP, part = (q % WP) ^ pf_wswz<FMT>(rl);
-    const int j = rl >> 4;
-    const DevWeight& w = (EPI == EPI_SWIGLU && j >= NQ) ? seg.w2 : seg.w;
-    int64_t r = n0 + 16 * (j % NQ) + (rl & 15);
-    r = mr.wrow0 + (r < seg.rows ? r : seg.rows - 1);
-    wsrc_q[u] = w.a + r * w.a_row + 16 * part;
-  }
-  const uint8_t* wsrc_s;
-  {
-    const int rl = lane & (NR - 1);
-    const int j = rl >> 4;
-    const DevWeight& w = (EPI == EPI_SWIGLU && j >= NQ) ? seg.w2 : seg.w;
-    int64_t r = n0 + 16 * (j % NQ) + (rl & 15);
-    r = mr.wrow0 + (r < seg.rows ? r : seg.rows - 1);
-    wsrc_s = w.b + r * w.b_row;
-  }
-
-  auto issue = [&](int stl, int slot) __attribute__((always_inline)) {
-    const int64_t st = sbase + stl;
-    uint8_t* base = lds + slot * SB;
-    // activations
-#pragma unroll
-    for (int u = 0; u < NA; ++u)
-      dma16s(uniform_ptr(abase + st * 128), aoff[u],
-             lds_addr(base + ((ablk * 2 + (wave & 1)) * BM + 16 * (asub0 + u)) * 64));
-    // weight payload and scales of this wave's rows
-    uint8_t* wb = base + dma_a_bytes<MT>() + wave * WB;
-#pragma unroll
-    for (int u = 0; u < NWQ; ++u) dma16(wsrc_q[u] + st * QB, lds_addr(wb + u * 1024));
-    dma4(wsrc_s + st * 4, lds_addr(wb + NR * QB));
-  };
-  auto wait_stage = [&](int st) __attribute__((always_inline)) {
-    // stage st is complete when at most the next stage's loads are outstanding
-    if (st + 1 < nst) __builtin_amdgcn_s_waitcnt(0x0f70 | ND);  // vmcnt(ND), lgkm/exp untouched
-    else __builtin_amdgcn_s_waitcnt(0x0f70);                    // vmcnt(0)
-    __builtin_amdgcn_s_barrier();
-  };
-
-  f4_t acc[MT][NT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-  auto compute = [&](int stl, int slot) __attribute__((always_inline)) {
-    const int64_t st = sbase + stl;
-    const uint8_t* base = lds + slot * SB;
-    const uint8_t* wb = base + dma_a_bytes<MT>() + wave * WB;
-    PfRaw<FMT> rw[NT];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      // block s of the row: part s (Q4_0: 16 bytes, lane half g & 1) or parts
-      // 2 s, 2 s + 1 (Q8_0: 32 bytes, lane quarter g)
-      const uint8_t* rowp = wb + (16 * j + col) * QB;
-#pragma unroll
-      for (int sb = 0; sb < 2; ++sb) {
-        const int part = (FMT == T_Q4_0) ? sb : 2 * sb + (g >> 1);
-        rw[j].q[sb] = *reinterpret_cast<const uint2*>(rowp + 16 * (part ^ pf_wswz<FMT>(col)) + 8 * (g & 1));
-      }
-      rw[j].d = *reinterpret_cast<const uint32_t*>(wb + NR * QB + 4 * (16 * j + col));
-    }
-    // Steps (block sb, subtile i) in order, each fenced from the next so that
-    // the registers live at once stay bounded: a step reads the next step's A
-    // fragments, issues its own matrix-core ops, then applies the previous
-    // step's block scales while those ops run.
-    auto afrag = [&](int sb, int i, h8_t& hi, h8_t& lo) __attribute__((always_inline)) {
-      const int r = 16 * i + col;
-      const int off = r * 64 + 16 * (g ^ pf_swz(r));
-      hi = *reinterpret_cast<const h8_t*>(base + ((sb * 2 + 0) * BM) * 64 + off);
-      lo = *reinterpret_cast<const h8_t*>(base + ((sb * 2 + 1) * BM) * 64 + off);
-    };
-    h8_t nhi, nlo;
-    afrag(0, 0, nhi, nlo);
-    f4_t pp[NT];
-    float psc[NT];
-    PfFrag<FMT> fr[NT];
-#pragma unroll
-    for (int sb = 0; sb < 2; ++sb) {
-#pragma unroll
-      for (int j = 0; j < NT; ++j) pf_decode<FMT, H16>(rw[j], st, sb, g, fr[j]);
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int step = sb * MT + i;
-        const h8_t ahi = nhi, alo = nlo;
-        if (step + 1 < 2 * MT) afrag((step + 1) / MT, (step + 1) % MT, nhi, nlo);
-        f4_t pc[NT];
-#pragma unroll
-        for (int j = 0; j < NT; ++j) pc[j] = mfma32(ahi, fr[j].b, f4_t{0.0f, 0.0f, 0.0f, 0.0f});
-#pragma unroll
-        for (int j = 0; j < NT; ++j) pc[j] = mfma32(alo, fr[j].b, pc[j]);
-        if (step > 0) {
-#pragma unroll
-          for (int j = 0; j < NT; ++j) acc[(step - 1) % MT][j] += psc[j] * pp[j];
-        }
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          pp[j] = pc[j];
-          psc[j] = fr[j].sc[0];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[MT - 1][j] += psc[j] * pp[j];
-  };
-
-  issue(0, 0);
-  if (nst > 1) issue(1, 1);
-  for (int st = 0; st < nst; st += 3) {
-    wait_stage(st);
-    if (st + 2 < nst) issue(st + 2, 2);
-    compute(st, 0);
-    if (st + 1 >= nst) break;
-    wait_stage(st + 1);
-    if (st + 3 < nst) issue(st + 3, 0);
-    compute(st + 1, 1);
-    if (st + 2 >= nst) break;
-    wait_stage(st + 2);
-    if (st + 4 < nst) issue(st + 4, 1);
-    compute(st + 2, 2);
-  }
-
-  // epilogue: lane holds rows m0 + 16i + 4g + r of column n0 + 16j + col
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t t = m0 + 16 * i + 4 * g + r;
-      if (t >= mr.mend) continue;
-      const float rs = a.rs[pf_arow(a, mr, t)];
-      float* yrow = a.y + t * a.ldy + seg.col0;
-#pragma unroll
-      for (int j = 0; j < NQ; ++j) {
-        const int64_t n = n0 + 16 * j + col;
-        if (n >= seg.rows) continue;
-        const float v = acc[i][j][r] * rs;
-        if constexpr (EPI == EPI_STORE) {
-          if (a.ksplit > 1) a.part[((int64_t)blockIdx.z * a.M + t) * a.ldy + seg.col0 + n] = v;
-          else yrow[n] = v;
-        } else if constexpr (EPI == EPI_ADD) {
-          if (a.ksplit > 1) a.part[((int64_t)blockIdx.z * a.M + t) * a.ldy + seg.col0 + n] = v;
-          else yrow[n] = yrow[n] + v;
-        } else if constexpr (EPI == EPI_SWIGLU) {
-          const float u = acc[i][j + NQ][r] * rs;
-          const float act = v / (1.0f + expf(-v));  // silu (elementwise.cpp:73-84)
-          yrow[n] = act * u;
-        } else if constexpr (EPI == EPI_GELU) {
-          const float inner = 0.7978845608f * (v + 0.044715f * v * v * v);
-          yrow[n] = 0.5f * v * (1.0f + tanhf(inner));
-        }
+        d[24] = (_Float16)0.0f;
       }
     }
   }
@@ -1556,187 +774,26 @@ __global__ void __launch_bounds__(256) k_pf_moe_combine(float* __restrict__ x, i
 
 // ---- launchers ------------------------------------------------------------------------------
 
-bool pf_supported(int type) {
-  return type == T_Q4_0 || type == T_Q8_0 || type == T_Q4_K || type == T_Q6_K;
-}
-
-int64_t pf_mpad(int64_t m) { return (m + 63) / 64 * 64; }
-
 bool pf_row_supported(int64_t K) { return K * 4 <= lds_limit() - 2048; }
 
 hipError_t launch_pf_prep(float* x, int64_t ldx, int64_t M, const float* norm_w, float eps,
                           const PfAct& act, hipStream_t s, const float* part, int nsplit) {
   if (nsplit < 0 || (nsplit > 0 && !part)) return hipErrorInvalidValue;
-  if (M <= 0 || M > act.mpad || act.K % 32 || act.mpad % 64 || ldx % 4) return hipErrorInvalidValue;
+  if (M <= 0 || M > act.mpad || act.K % 32 || act.mpad != pf_mpad(act.mpad) || ldx % 4 || (act.sxp && act.K % 256))
+    return hipErrorInvalidValue;
   const size_t lds = (size_t)act.K * 4;
   if ((int64_t)lds > lds_limit()) return hipErrorInvalidValue;
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_prep),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-  }
-  UAII_LAUNCH(k_pf_prep, dim3((unsigned)act.mpad), dim3(256), lds, s, x, ldx, M, norm_w, eps, act,
-              part, nsplit);
-  return hipGetLastError();
-}
-
-namespace {
-template <int FMT, int EPI, int MT, int NT>
-hipError_t pf_gemm_go(PfGemmArgs a, hipStream_t s) {
-  const int per_tile = PF_WAVES * 16 * (EPI == EPI_SWIGLU ? NT / 2 : NT);
-  int ntiles = 0;
-  for (int k = 0; k < a.nseg; ++k) {
-    a.seg[k].tile0 = ntiles;
-    ntiles += (int)((a.seg[k].rows + per_tile - 1) / per_tile);
-  }
-  if (a.gtab && a.gbm != 16 * MT) return hipErrorInvalidValue;
-  dim3 grid((unsigned)ntiles, (unsigned)(a.gtab ? a.ntab : a.mpad / (16 * MT)), (unsigned)a.ksplit);
-  UAII_LAUNCH((k_pf_gemm<FMT, EPI, MT, NT>), grid, dim3(PF_WAVES * 64), 0, s, a);
-  return hipGetLastError();
-}
-
-template <int FMT, int EPI, int MT>
-hipError_t pf_gemm_dma_go(PfGemmArgs a, hipStream_t s) {
-  constexpr int NT = dma_nt<FMT>();
-  const int per_tile = PF_DW * 16 * (EPI == EPI_SWIGLU ? NT / 2 : NT);
-  int ntiles = 0;
-  for (int k = 0; k < a.nseg; ++k) {
-    a.seg[k].tile0 = ntiles;
-    ntiles += (int)((a.seg[k].rows + per_tile - 1) / per_tile);
-  }
-  if (a.gtab && a.gbm != 16 * MT) return hipErrorInvalidValue;
-  dim3 grid((unsigned)ntiles, (unsigned)(a.gtab ? a.ntab : a.mpad / (16 * MT)), (unsigned)a.ksplit);
-  if constexpr (FMT == T_Q4_0) {
-    if (a.hi16) {
-      UAII_LAUNCH((k_pf_gemm_dma<FMT, EPI, MT, NT, true>), grid, dim3(PF_DW * 64), 0, s, a);
-      return hipGetLastError();
+  auto go = [&](auto kernel, int threads) -> hipError_t {
+    if (lds > 64 * 1024) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return e;
     }
-  }
-  UAII_LAUNCH((k_pf_gemm_dma<FMT, EPI, MT, NT, false>), grid, dim3(PF_DW * 64), 0, s, a);
-  return hipGetLastError();
-}
-
-// Wave tile per launch: 64 x 32 (measured best at M = 512 for the 8B shapes,
-// ahead of 64 x 64 and 32 x 32; for Q4_K 232 against 196 TFLOP/s on the 1B
-// gate/up; for Q6_K 85 against 67 TFLOP/s on the 1B down with the former
-// 16x16x16 decode) unless that leaves the grid under one block per CU; then
-// 32 x 32.
-template <int FMT, int EPI>
-hipError_t pf_gemm_tile(const PfGemmArgs& a, hipStream_t s) {
-  int64_t rows = 0;
-  for (int k = 0; k < a.nseg; ++k) rows += a.seg[k].rows;
-  if (EPI == EPI_SWIGLU) rows *= 2;
-  const int64_t mid = (rows / 128) * (a.mpad / 64);
-  constexpr bool wide = FMT == T_Q4_0 || FMT == T_Q8_0;
-  const int want = UAII_PF_TILE;
-  if (a.gtab) {  // expert groups: the tile height their table was built for
-    if constexpr (wide) {
-      if (UAII_PF_DMA) return pf_gemm_dma_go<FMT, EPI, 4>(a, s);
-      return pf_gemm_go<FMT, EPI, 4, 2>(a, s);
-    }
-    if constexpr (FMT == T_Q4_K) {
-      if (UAII_PF_KTILE) return pf_gemm_go<FMT, EPI, 4, 2>(a, s);
-    }
-    return pf_gemm_go<FMT, EPI, 2, 2>(a, s);
-  }
-  if constexpr (wide) {
-    if (UAII_PF_DMA) {
-      if (want == 2 || (want == 0 && mid >= 256)) return pf_gemm_dma_go<FMT, EPI, 4>(a, s);
-      return pf_gemm_dma_go<FMT, EPI, 2>(a, s);
-    }
-    if (want == 2 || (want == 0 && mid >= 256)) return pf_gemm_go<FMT, EPI, 4, 2>(a, s);
-  }
-  if constexpr (FMT == T_Q4_K) {
-    if (UAII_PF_KTILE && (want == 2 || (want == 0 && mid >= 256))) return pf_gemm_go<FMT, EPI, 4, 2>(a, s);
-  }
-  if constexpr (FMT == T_Q6_K) {
-    if (UAII_PF_K6TILE && (want == 2 || (want == 0 && mid >= 256))) return pf_gemm_go<FMT, EPI, 4, 2>(a, s);
-  }
-  return pf_gemm_go<FMT, EPI, 2, 2>(a, s);
-}
-
-template <int FMT>
-hipError_t pf_gemm_epi(const PfGemmArgs& a, hipStream_t s) {
-  switch (a.epi) {
-    case EPI_STORE: return pf_gemm_tile<FMT, EPI_STORE>(a, s);
-    case EPI_ADD: return pf_gemm_tile<FMT, EPI_ADD>(a, s);
-    case EPI_SWIGLU: return pf_gemm_tile<FMT, EPI_SWIGLU>(a, s);
-    case EPI_GELU: return pf_gemm_tile<FMT, EPI_GELU>(a, s);
-    default: return hipErrorInvalidValue;
-  }
-}
-}  // namespace
-
-// K split for a residual-add or plain-store launch: enough blocks for two per CU
-// (each block's K range a whole number of stages and, for the K-quants,
-// super-blocks).
-int pf_gemm_ksplit(const PfGemmArgs& a, int cus) {
-  if ((a.epi != EPI_ADD && a.epi != EPI_STORE) || a.nseg < 1) return 1;
-  const int type = a.seg[0].w.type;
-  if (!pf_supported(type)) return 1;
-  int64_t rows = 0;
-  for (int k = 0; k < a.nseg; ++k) rows += a.seg[k].rows;
-  const bool wide = type == T_Q4_0 || type == T_Q8_0;
-  const bool tall = wide || (type == T_Q4_K && UAII_PF_KTILE);  // formats with the 64 x 32 wave tile
-  const int64_t mid = (rows / 128) * (a.mpad / 64);
-  const bool big_tile = tall && (UAII_PF_TILE == 2 || (UAII_PF_TILE == 0 && mid >= 256));
-  const int nw = (wide && UAII_PF_DMA) ? PF_DW : PF_WAVES;  // waves per block
-  const int64_t tiles = (rows + nw * 32 - 1) / (nw * 32);     // 32 weight rows per wave
-  const int64_t blocks = tiles * (a.mpad / (big_tile ? 64 : 32));
-  const int64_t kq = wide ? 64 : 256;
-  int ks = 1;
-  const int64_t want = (int64_t)cus * UAII_PF_KS_BPC * PF_WAVES / nw;  // blocks (of PF_WAVES-wave units)
-  while (ks < 4 && blocks * ks < want && a.K % (kq * ks * 2) == 0) ks *= 2;
-  return ks;
-}
-
-int pf_gemm_group_rows(int type) {
-  return (type == T_Q4_0 || type == T_Q8_0 || (type == T_Q4_K && UAII_PF_KTILE)) ? 64 : 32;
-}
-
-bool pf_hi16_supported(int type) { return type == T_Q4_0 && UAII_PF_DMA; }
-
-hipError_t launch_pf_gemm(PfGemmArgs a, hipStream_t s) {
-  if (a.ksplit < 1) a.ksplit = 1;
-  if (a.sx_ld <= 0) a.sx_ld = a.mpad;
-  if (!a.arow && !a.gtab && a.sx_ld != a.mpad) return hipErrorInvalidValue;
-  if (a.nseg < 1 || a.nseg > 3 || a.M <= 0 || a.M > a.mpad || a.mpad % 64 || a.K % 64)
-    return hipErrorInvalidValue;
-  if (a.gtab) {
-    // every table entry lies inside [0, M) and names an expert below ngroups (the
-    // caller builds it on the host); here the launch itself is checked
-    if (a.ntab < 1 || a.ngroups < 1 || a.ksplit != 1 || a.nseg != 1 ||
-        a.gbm != pf_gemm_group_rows(a.seg[0].w.type) || (!a.arow && a.sx_ld < a.mpad))
-      return hipErrorInvalidValue;
-    const PfSeg& sg = a.seg[0];
-    if (sg.rows * a.ngroups > sg.w.rows || (a.epi == EPI_SWIGLU && sg.rows * a.ngroups > sg.w2.rows))
-      return hipErrorInvalidValue;
-  }
-  const int type = a.seg[0].w.type;
-  if (!pf_supported(type)) return hipErrorInvalidValue;
-  // the direct-to-LDS kernels (Q4_0, Q8_0) address activation rows by 32-bit
-  // byte offsets: their activation arrays must span under 2^31 bytes
-  if ((type == T_Q4_0 || type == T_Q8_0) && UAII_PF_DMA && a.sx_ld * a.K * 2 >= (int64_t(1) << 31))
-    return hipErrorInvalidValue;
-  if (a.hi16 && !pf_hi16_supported(type)) return hipErrorInvalidValue;
-  const int64_t kq = (type == T_Q4_K || type == T_Q6_K) ? 256 : 64;  // K granule of a block's range
-  if (a.K % (kq * a.ksplit)) return hipErrorInvalidValue;
-  if (a.ksplit > 1 && ((a.epi != EPI_ADD && a.epi != EPI_STORE) || !a.part)) return hipErrorInvalidValue;
-  for (int k = 0; k < a.nseg; ++k) {
-    const PfSeg& sg = a.seg[k];
-    if (sg.w.type != type || sg.w.cols != a.K || sg.rows <= 0 || sg.rows > sg.w.rows)
-      return hipErrorInvalidValue;
-    if (a.epi == EPI_SWIGLU &&
-        (sg.w2.type != type || sg.w2.cols != a.K || sg.rows > sg.w2.rows))
-      return hipErrorInvalidValue;
-  }
-  switch (type) {
-    case T_Q4_0: return pf_gemm_epi<T_Q4_0>(a, s);
-    case T_Q8_0: return pf_gemm_epi<T_Q8_0>(a, s);
-    case T_Q4_K: return pf_gemm_epi<T_Q4_K>(a, s);
-    case T_Q6_K: return pf_gemm_epi<T_Q6_K>(a, s);
-    default: return hipErrorInvalidValue;
-  }
+    UAII_LAUNCH(kernel, dim3((unsigned)act.mpad), dim3(threads), lds, s, x, ldx, M, norm_w, eps, act, part, nsplit);
+    return hipGetLastError();
+  };
+  // up to a block per two CUs the row's own latency is the launch's
+  return act.mpad <= 128 && act.K >= 1024 ? go(&k_pf_prep<1024>, 1024) : go(&k_pf_prep<256>, 256);
 }
 
 hipError_t launch_pf_qkv(const PfQkvArgs& a, hipStream_t s) {

@@ -247,19 +247,20 @@ hipError_t launch_argmax_final(float* part_val, int32_t* part_idx, int nparts, S
 
 // ---- prefill (M > 1 prompt tokens, matrix cores) ---------------------------------------
 
-// Activation rows prepared for the MFMA GEMM: x * 2^e = hi + lo in f16 (each
-// aligned group of 4 stored as k0, k2, k1, k3), per-32 sums of x * 2^e, and 2^-e.
+// Activation rows prepared for the row GEMMs: x * 2^e = hi + lo in f16, and 2^-e.
+// One 32-block of all rows after another ([K / 32][mpad][32], so that 16 rows of a
+// block are one contiguous kilobyte), a block's quads in the order 0, 4, 1, 5, 2, 6,
+// 3, 7 and each quad as k0, k2, k1, k3: the order in which the weights' bytes
+// decode (prefill_gemm.hip). sxp: per 256 k a block of the same shape holding the
+// sums of x * 2^(e - 5) over the eight 32-blocks as f16 parts (eight first parts,
+// eight second, eight third, eight zeros; together all 24 bits).
 struct PfAct {
-  __half* hi;     // [mpad][K]
-  __half* lo;     // [mpad][K]
-  float* sx;      // [K / 32][mpad]
+  __half* hi;
+  __half* lo;
+  __half* sxp;    // [K / 256][mpad][32], or null where no consumer takes it
   float* rs;      // [mpad]
-  int64_t mpad;   // rows allocated (multiple of 64); rows >= M are zero
+  int64_t mpad;   // rows allocated (pf_mpad); rows >= M are zero
   int64_t K;
-  // 1: the layout the Q4_0 direct-to-LDS GEMM takes with its high nibbles
-  // decoded in place (elements 16..31 of every 32-block stored times 1/16);
-  // only for activations every consumer of which is such a launch
-  int hi16;
 };
 
 struct PfSeg {
@@ -277,26 +278,26 @@ struct PfGemmArgs {
   int64_t M, K, mpad;
   const __half* ahi;
   const __half* alo;
-  const float* sx;
+  const __half* sxp;    // Q4_K, Q5_K
   const float* rs;
   float* y;             // [M][ldy]
   int64_t ldy;
-  // EPI_ADD split over K: ksplit > 1 blocks along grid z each take K / ksplit
-  // and store their partial to part[z][M][ldy] instead of adding into y; the
-  // next launch_pf_prep of y adds the partials (z in order) into y
+  // ksplit > 1: blocks along grid z each take a share of K and store their sums to
+  // part[z][M][ldp] (EPI_SWIGLU: gate and up sums side by side) instead of the
+  // epilogue, which launch_pf_fold or the next kernel to read y does, z in order
   int ksplit;
   float* part;
+  int64_t ldp;
   // optional activation-row map: output row t reads activation row arow[t]
-  // (MoE experts gather their tokens); rows are those of ahi/alo/sx/rs
+  // (MoE experts gather their tokens); rows are those of ahi/alo/sxp/rs
   const int32_t* arow;
-  int64_t sx_ld;  // row stride of sx (the activations' padded row count); 0: mpad
+  int64_t act_ld;  // the activations' padded row count; 0: mpad
   // optional expert grouping (MoE): grid row y computes output rows
   // [gtab[3y + 1], gtab[3y + 2]) against expert gtab[3y] of the weight stacks,
   // whose rows e * seg.rows .. (e + 1) * seg.rows - 1 are that expert's;
   // at most gbm rows per entry (pf_gemm_group_rows of the format)
   const int32_t* gtab;
   int ntab, ngroups, gbm;
-  int hi16;       // the activations carry PfAct::hi16's layout (Q4_0 only)
 };
 
 struct PfQkvArgs {
@@ -345,6 +346,10 @@ hipError_t launch_pf_moe_combine(float* x, int64_t M, int64_t D, int k, const fl
 bool pf_router_supported(int type);
 
 bool pf_supported(int type);
+bool pf_k_quant(int type);  // rows are whole 256-value super-blocks
+// The formats that prefill() takes and whose row GEMM reports what it cannot run; the
+// others' callers ran token by token or row by row before, and fall back to that.
+bool pf_required(int type);
 bool pf_attn_supported(int head_dim, int n_heads, int n_kv);
 int64_t pf_mpad(int64_t m);
 // Whether launch_pf_prep (and the MoE routing) can stage a row of K values.
@@ -354,11 +359,12 @@ bool pf_row_supported(int64_t K);
 hipError_t launch_pf_prep(float* x, int64_t ldx, int64_t M, const float* norm_w, float eps,
                           const PfAct& act, hipStream_t s, const float* part = nullptr,
                           int nsplit = 0);
-// Whether a weight format's prefill GEMM takes PfAct::hi16 activations.
-bool pf_hi16_supported(int type);
 hipError_t launch_pf_gemm(PfGemmArgs a, hipStream_t s);
-// K split launch_pf_gemm can take for `a` (EPI_ADD only; 1 = none) on `cus` CUs.
-int pf_gemm_ksplit(const PfGemmArgs& a, int cus);
+int pf_device_cus();
+// K split for `a` on `cus` CUs whose partials fit part_floats (1 = none).
+int pf_gemm_ksplit(const PfGemmArgs& a, int cus, int64_t part_floats);
+// The partials of a K-split launch into y through its epilogue (one segment).
+hipError_t launch_pf_fold(const PfGemmArgs& a, hipStream_t s);
 // rows per entry of an expert-grouped GEMM's table for this block format
 int pf_gemm_group_rows(int type);
 hipError_t launch_pf_qkv(const PfQkvArgs& a, hipStream_t s);

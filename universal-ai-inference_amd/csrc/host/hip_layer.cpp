@@ -179,7 +179,7 @@ int gemm_common(const uaii_hip_weight* w, const uaii_hip_weight* w2, const float
     if (u.type != v.type || u.rows != v.rows || u.cols != v.cols) return kErrArg;
   }
   const int64_t K = v.cols, N = v.rows;
-  if (!pf_supported(v.type) || K % 64) {
+  auto row_by_row = [&]() -> int {
     for (int64_t i = 0; i < m; ++i) {
       const float* xi = x + i * K;
       float* yi = y + i * N;
@@ -189,41 +189,72 @@ int gemm_common(const uaii_hip_weight* w, const uaii_hip_weight* w2, const float
       if (rc) return rc;
     }
     return 0;
-  }
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
+  };
+  // Formats that used to run row by row still do where the row path's row length,
+  // grid or memory ends; the others report it.
+  const bool required = pf_required(v.type);
+  if (!pf_supported(v.type) || K % 64) return row_by_row();
+  if (!required && (!pf_row_supported(K) || m > 65535 * 64)) return row_by_row();
+  std::unique_lock<std::mutex> lk(g_scratch_mu);
   const int64_t mpad = pf_mpad(m);
-  const size_t hb = (size_t)mpad * (size_t)K * 2, sxb = (size_t)(K / 32) * (size_t)mpad * 4;
-  int rc = grow_scratch(2 * hb + sxb + (size_t)mpad * 4);
-  if (rc) return rc;
-  char* base = static_cast<char*>(g_scratch);
-  PfAct act{};
-  act.hi = reinterpret_cast<__half*>(base);
-  act.lo = reinterpret_cast<__half*>(base + hb);
-  act.sx = reinterpret_cast<float*>(base + 2 * hb);
-  act.rs = reinterpret_cast<float*>(base + 2 * hb + sxb);
-  act.mpad = mpad;
-  act.K = K;
-  act.hi16 = pf_hi16_supported(v.type) ? 1 : 0;  // this launch is the activations' only consumer
-  hipError_t e = launch_pf_prep(const_cast<float*>(x), K, m, norm_w, eps, act, S(stream));
-  if (e != hipSuccess) return (int)e;
   PfGemmArgs a{};
   a.nseg = 1;
   a.epi = epi;
   a.M = m;
   a.K = K;
   a.mpad = mpad;
-  a.ahi = act.hi;
-  a.alo = act.lo;
-  a.sx = act.sx;
-  a.rs = act.rs;
   a.y = y;
   a.ldy = N;
   a.seg[0].w = v;
   if (w2) a.seg[0].w2 = w2->w.view;
   a.seg[0].rows = N;
   a.seg[0].col0 = 0;
-  a.hi16 = act.hi16;
-  return (int)launch_pf_gemm(a, S(stream));
+  // A launch that leaves the chip idle splits K; its partials, kept to 64 MB, are
+  // folded by one more launch.
+  a.ksplit = pf_gemm_ksplit(a, pf_device_cus(), (int64_t)16 << 20);
+  a.ldp = epi == EPI_SWIGLU ? 2 * N : N;
+  const size_t hb = (size_t)mpad * (size_t)K * 2, xb = K % 256 == 0 ? hb / 8 : 0, rb = (size_t)mpad * 4;
+  auto reserve = [&]() -> int {
+    const size_t pb = a.ksplit > 1 ? (size_t)a.ksplit * (size_t)m * (size_t)a.ldp * 4 : 0;
+    const size_t need = 2 * hb + xb + rb + pb;
+    if (need <= g_scratch_bytes) return 0;
+    // growing allocates, which a captured stream does not allow
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (stream && (a.ksplit > 1 || !required) && hipStreamIsCapturing(S(stream), &cs) == hipSuccess &&
+        cs != hipStreamCaptureStatusNone)
+      return (int)hipErrorStreamCaptureUnsupported;
+    return grow_scratch(need);
+  };
+  int rc = reserve();
+  if (rc && a.ksplit > 1) {
+    (void)hipGetLastError();
+    a.ksplit = 1;
+    rc = reserve();
+  }
+  if (rc && !required) {
+    (void)hipGetLastError();
+    lk.unlock();
+    return row_by_row();
+  }
+  if (rc) return rc;
+  char* base = static_cast<char*>(g_scratch);
+  PfAct act{};
+  act.hi = reinterpret_cast<__half*>(base);
+  act.lo = reinterpret_cast<__half*>(base + hb);
+  act.sxp = (v.type == T_Q4_K || v.type == T_Q5_K) ? reinterpret_cast<__half*>(base + 2 * hb) : nullptr;
+  act.rs = reinterpret_cast<float*>(base + 2 * hb + xb);
+  act.mpad = mpad;
+  act.K = K;
+  hipError_t e = launch_pf_prep(const_cast<float*>(x), K, m, norm_w, eps, act, S(stream));
+  if (e != hipSuccess) return (int)e;
+  a.ahi = act.hi;
+  a.alo = act.lo;
+  a.sxp = act.sxp;
+  a.rs = act.rs;
+  a.part = reinterpret_cast<float*>(base + 2 * hb + xb + rb);
+  e = launch_pf_gemm(a, S(stream));
+  if (e != hipSuccess || a.ksplit <= 1) return (int)e;
+  return (int)launch_pf_fold(a, S(stream));
 }
 
 }  // namespace

@@ -345,6 +345,7 @@ Error DecoderProgram::build(const DecoderSpec& spec, const ProgramOptions& opts)
   // attention takes
   bool rows = pf_attn_supported((int)d.head_dim, (int)d.n_heads, (int)d.n_kv_heads) && d.dim % 64 == 0 &&
               d.q_dim % 64 == 0;
+  bool required = true;
   for (int64_t li = 0; rows && li < d.n_layers; ++li) {
     const Layer& L = *layers_[(size_t)li];
     const LayerSpec& ls = d.layers[(size_t)li];
@@ -360,12 +361,15 @@ Error DecoderProgram::build(const DecoderSpec& spec, const ProgramOptions& opts)
       if (!pf_router_supported(L.gate_inp.view.type)) rows = false;
     }
     if (ls.ffn != LayerSpec::kNone && ls.inter % 64) rows = false;
-    for (const DeviceWeight* w : ws) rows = rows && pf_supported(w->view.type);
+    for (const DeviceWeight* w : ws) {
+      rows = rows && pf_supported(w->view.type);
+      required = required && pf_required(w->view.type);
+    }
   }
   if (const char* env = std::getenv("UAII_PREFILL")) {
     if (std::string(env) == "0") rows = false;
   }
-  pf_ok_ = rows && opts_.kv_f16;
+  pf_ok_ = rows && required && opts_.kv_f16;
   pf_rows_ = rows;
   // a row longer than the prep stages runs in token steps (prefill() reports it)
   if (!pf_ok_) {
@@ -373,9 +377,6 @@ Error DecoderProgram::build(const DecoderSpec& spec, const ProgramOptions& opts)
     for (const LayerSpec& ls : d.layers) pf_rows_ = pf_rows_ && pf_row_supported(ls.inter);
     for (const auto& L : layers_) pf_rows_ = pf_rows_ && pf_row_supported(L->inter_sh);
   }
-  // Q4_0 GEMMs take their high nibbles in place (PfAct::hi16) where every
-  // consumer of a prep is one; UAII_PF_H16=0 keeps the shifted decode
-  if (const char* env = std::getenv("UAII_PF_H16")) pf_h16_ = std::string(env) != "0";
   UAII_TRY(alloc(1024, (void**)&ring_pad_));
   {
     // the ring kernel measures faster for the residual-add GEMVs (O, down; the
@@ -429,8 +430,12 @@ Error DecoderProgram::ensure_prefill_buffers(int64_t chunk) {
   UAII_TRY(alloc(4 * C * (size_t)d.q_dim, (void**)&pf_attn_));
   UAII_TRY(alloc(4 * C * (size_t)inter, (void**)&pf_h_));
   // K-split partials: the residual stream's, or the QKV group's
-  pf_part_cols_ = std::max(d.dim, d.q_dim + 2 * d.kv_dim);
-  UAII_TRY(alloc(4 * 4 * C * (size_t)pf_part_cols_, (void**)&pf_part_));
+  // (and, in short chunks, what feeds the down projection): 4 splits of a chunk's
+  // rows, more in short chunks unless the session has a byte budget to keep
+  pf_part_floats_ = 4 * chunk * std::max(d.dim, d.q_dim + 2 * d.kv_dim);
+  if (opts_.budget_bytes == 0)
+    pf_part_floats_ = std::max<int64_t>(pf_part_floats_, std::min<int64_t>(chunk, 64) * 16 * std::max(d.q_dim + 2 * d.kv_dim, 2 * inter));
+  UAII_TRY(alloc(4 * (size_t)pf_part_floats_, (void**)&pf_part_));
   if (moe_) {
     const size_t CK = C * (size_t)topk;
     UAII_TRY(alloc(4 * CK, (void**)&pf_moe_ids_));
@@ -450,7 +455,7 @@ Error DecoderProgram::ensure_prefill_buffers(int64_t chunk) {
   }
   UAII_TRY(alloc(2 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.hi));
   UAII_TRY(alloc(2 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.lo));
-  UAII_TRY(alloc(4 * (size_t)(kmax / 32) * (size_t)mpad, (void**)&pf_act_.sx));
+  UAII_TRY(alloc(64 * (size_t)((kmax + 255) / 256) * (size_t)mpad, (void**)&pf_act_.sxp));
   UAII_TRY(alloc(4 * (size_t)mpad, (void**)&pf_act_.rs));
   pf_act_.mpad = mpad;
   pf_act_rows_ = mpad;
@@ -472,11 +477,10 @@ Error DecoderProgram::pf_gemm(const DeviceWeight* w[3], const int64_t cols0[3], 
     a.mpad = pf_act_.mpad;
     a.ahi = pf_act_.hi;
     a.alo = pf_act_.lo;
-    a.sx = pf_act_.sx;
+    a.sxp = pf_act_.sxp;
     a.rs = pf_act_.rs;
     a.y = y;
     a.ldy = ldy;
-    a.hi16 = pf_act_.hi16;
     int j = i;
     while (j < nw && w[j]->view.type == w[i]->view.type) {
       PfSeg& sg = a.seg[a.nseg++];
@@ -491,27 +495,27 @@ Error DecoderProgram::pf_gemm(const DeviceWeight* w[3], const int64_t cols0[3], 
       UAII_HIP(hipGetDevice(&dev));
       UAII_HIP(hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, dev));
     }
-    // a residual add into the stream of a single-format launch may split K; its
-    // partials are added by the next prep of the stream (pf_prep)
+    // A launch that leaves the chip idle splits K. A residual add into the stream
+    // leaves its partials to the next prep of the stream (pf_prep), a split store
+    // to its reader (every launch of the group writes the same split); what feeds
+    // the down projection is folded here.
+    const bool stream_add = epi == EPI_ADD && y == pf_x_ && i == 0 && j == nw && pf_pending_ == 0;
+    const bool fold = (epi == EPI_SWIGLU || epi == EPI_GELU) && nw == 1;
     a.ksplit = 1;
-    if (epi == EPI_ADD && y == pf_x_ && i == 0 && j == nw && pf_pending_ == 0) {
-      a.ksplit = pf_gemm_ksplit(a, cus_);
-      a.part = pf_part_;
-    }
-    // a split store: every launch of the group writes partials with the same split
-    if (store_split > 1) {
-      a.ksplit = store_split;
-      a.part = pf_part_;
-    }
+    a.part = pf_part_;
+    a.ldp = epi == EPI_SWIGLU ? 2 * a.seg[0].rows : fold ? a.seg[0].rows : ldy;
+    if (store_split > 1) a.ksplit = store_split;
+    else if (stream_add || fold) a.ksplit = pf_gemm_ksplit(a, cus_, pf_part_floats_);
     UAII_HIP(launch_pf_gemm(a, stream_));
-    if (epi == EPI_ADD && a.ksplit > 1) pf_pending_ = a.ksplit;
+    if (a.ksplit > 1 && fold) UAII_HIP(launch_pf_fold(a, stream_));
+    if (a.ksplit > 1 && stream_add) pf_pending_ = a.ksplit;
     i = j;
   }
   return Error::success();
 }
 
-// K split shared by the launches of a plain-store group (QKV): the largest any
-// launch of the group asks for, halved until every launch's K range allows it.
+// K split shared by the launches of a plain-store group (QKV): the smallest that a
+// launch of the group asks for.
 int DecoderProgram::pf_store_split(const DeviceWeight* w[3], int nw, int64_t m, int64_t ldy) {
   if (cus_ == 0) {
     int dev = 0;
@@ -519,9 +523,7 @@ int DecoderProgram::pf_store_split(const DeviceWeight* w[3], int nw, int64_t m, 
         hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       return 1;
   }
-  if ((int64_t)4 * pf_chunk_ * pf_part_cols_ < 4 * m * ldy) return 1;
-  int ks = 1;
-  int64_t kq = 64;
+  int ks = 1 << 16;
   for (int i = 0; i < nw;) {
     PfGemmArgs a{};
     a.epi = EPI_STORE;
@@ -535,23 +537,21 @@ int DecoderProgram::pf_store_split(const DeviceWeight* w[3], int nw, int64_t m, 
       sg.rows = w[j]->view.rows;
       ++j;
     }
-    const int t = w[i]->view.type;
-    if (t == T_Q4_K || t == T_Q6_K) kq = 256;
-    ks = std::max(ks, pf_gemm_ksplit(a, cus_));
+    // the launches run one after another, and the widest fills the chip first
+    const int k = pf_gemm_ksplit(a, cus_, pf_part_floats_);
+    ks = i == 0 ? k : std::min(ks, k);
     i = j;
   }
-  const int64_t K = w[0]->view.cols;
-  while (ks > 1 && K % (kq * ks) != 0) ks /= 2;
-  return ks;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(ks, pf_part_floats_ / std::max<int64_t>(m * ldy, 1)));
 }
 
-Error DecoderProgram::pf_prep(float* x, int64_t K, int64_t m, const float* norm_w, bool hi16) {
+Error DecoderProgram::pf_prep(float* x, int64_t K, int64_t m, const float* norm_w, bool sums) {
   if (pf_mpad(m) > pf_act_rows_ || K > pf_kmax_)
     return Error::make(ErrorCode::Internal, "prefill activation rows exceed their buffer");
   pf_act_.mpad = pf_mpad(m);
-  pf_act_.hi16 = hi16 ? 1 : 0;  // the GEMMs that read these rows take the same layout
   PfAct act = pf_act_;
   act.K = K;
+  if (!sums) act.sxp = nullptr;
   const int pend = (x == pf_x_) ? pf_pending_ : 0;
   UAII_HIP(launch_pf_prep(x, K, m, norm_w, spec_.rms_eps, act, stream_, pend ? pf_part_ : nullptr, pend));
   if (pend) pf_pending_ = 0;
@@ -570,7 +570,8 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
   const int E = (int)d.n_experts;
   const int k = (int)std::min<int64_t>(d.top_k, d.n_experts);
   const int64_t I = ls.inter;
-  UAII_TRY(prep(pf_x_, d.dim, m, L.ffn_norm));
+  auto sums = [](const DeviceWeight& w) { return w.view.type == T_Q4_K || w.view.type == T_Q5_K; };
+  UAII_TRY(prep(pf_x_, d.dim, m, L.ffn_norm, sums(L.gate_exps) || (L.shared && sums(L.gate_sh))));
   UAII_TRY(timed("pf_moe_route", 4.0 * (double)(m * d.dim + E * d.dim), 2.0 * (double)(m * E * d.dim), [&] {
     return launch_pf_moe_route(pf_x_, m, d.dim, L.ffn_norm, d.rms_eps, L.gate_inp.view, E, k, pf_moe_ids_,
                                pf_moe_w_, s);
@@ -617,9 +618,9 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
     g.mpad = pf_mpad(m * k);
     g.ahi = pf_act_.hi;
     g.alo = pf_act_.lo;
-    g.sx = pf_act_.sx;
+    g.sxp = pf_act_.sxp;
     g.rs = pf_act_.rs;
-    g.sx_ld = pf_act_.mpad;
+    g.act_ld = pf_act_.mpad;
     g.gtab = pf_moe_tab_ + 3 * t0;
     g.ntab = nt;
     g.ngroups = E;
@@ -644,7 +645,7 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
     UAII_TRY(gemm("pf_gemm_shared_gate_up", wg, c00, 1, &L.up_sh, EPI_SWIGLU, m, pf_hsh_, L.inter_sh));
   }
   // the routed tokens' hidden rows, packed by expert
-  UAII_TRY(prep(pf_h_, I, m * k, nullptr));
+  UAII_TRY(prep(pf_h_, I, m * k, nullptr, sums(L.down_exps)));
   {
     PfGemmArgs g = grouped(I, EPI_STORE, bm_dn, t_dn, n_dn);
     g.y = pf_moe_y_;
@@ -658,7 +659,7 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
     return launch_pf_moe_combine(pf_x_, m, d.dim, k, pf_moe_w_, pf_moe_inv_, pf_moe_y_, s);
   }));
   if (L.shared) {
-    UAII_TRY(prep(pf_hsh_, L.inter_sh, m, nullptr));
+    UAII_TRY(prep(pf_hsh_, L.inter_sh, m, nullptr, sums(L.down_sh)));
     const DeviceWeight* wd[3] = {&L.down_sh, nullptr, nullptr};
     UAII_TRY(gemm("pf_gemm_shared_down", wd, c00, 1, nullptr, EPI_ADD, m, pf_x_, d.dim));
   }
@@ -682,15 +683,20 @@ Error DecoderProgram::prefill(int64_t n) {
 Error DecoderProgram::generate_rows(int64_t n, bool* done) {
   *done = false;
   if (n <= 0 || !pf_rows_) return Error::success();
+  // A few tokens are faster in steps: the row path's launches cost what four captured
+  // steps do (prompts of 2, 4, 6 tokens, rows and steps in ms: 4-layer Q8_0 shape
+  // 0.46, 0.47, 0.49 and 0.29, 0.47, 0.66; 1B Q4_K shape 2.5, 2.6, 2.6 and 1.4, 2.7, 4.0).
+  const bool few = n < 4;
   if (pf_ok_) {
+    if (few) {
+      // a budget without room for the rows' buffers is refused as for any prompt
+      if (opts_.budget_bytes != 0) UAII_TRY(ensure_prefill_buffers(prefill_chunk(n)));
+      return Error::success();
+    }
     *done = true;
     return prefill_rows(n);
   }
-  // A few tokens are faster in steps: the layers' launches of the row path cost
-  // what 3 to 5 captured steps do (prompt of 4 / 6 tokens, f32 cache: 0.49 / 0.50
-  // against 0.49 / 0.69 ms on the 4-layer Q8_0 shape, 4.0 / 4.0 against 2.7 / 4.0
-  // ms on the 1B one).
-  if (n < 5) return Error::success();
+  if (few) return Error::success();
   // Such a session ran its prompt in token steps before this path took it, so
   // it must not need the path's buffers: without the memory it still does.
   if (!ensure_prefill_buffers(prefill_chunk(n)).ok()) {
@@ -715,10 +721,10 @@ Error DecoderProgram::prefill_rows(int64_t n) {
   const size_t layer_kv = (size_t)d.kv_dim * (size_t)max_ctx_ * (opts_.kv_f16 ? 2 : 4);
   const int64_t ldqkv = d.q_dim + 2 * d.kv_dim;
   prof_used_ = 0;
-  auto prep = [&](float* x, int64_t K, int64_t m, const float* norm_w, bool hi16 = false) -> Error {
+  auto prep = [&](float* x, int64_t K, int64_t m, const float* norm_w, bool sums) -> Error {
     Error err = Error::success();
     Error launched = timed("pf_prep", 12.0 * (double)m * (double)K, 0.0, [&]() -> hipError_t {
-      err = pf_prep(x, K, m, norm_w, hi16);
+      err = pf_prep(x, K, m, norm_w, sums);
       return err.ok() ? hipSuccess : hipErrorInvalidValue;
     });
     if (!err.ok()) return err;
@@ -763,10 +769,10 @@ Error DecoderProgram::prefill_rows(int64_t n) {
       const LayerSpec& ls = d.layers[(size_t)li];
       uint8_t* kbase = static_cast<uint8_t*>(kv_) + (size_t)li * 2 * layer_kv;
       uint8_t* vbase = kbase + layer_kv;
-      // each prep's layout: PfAct::hi16 when every GEMM reading it takes it
-      auto h16 = [&](const DeviceWeight& w) { return pf_h16_ && pf_hi16_supported(w.view.type); };
+      // a prep's per-32 sums, where a GEMM reading it takes them
+      auto sums = [](const DeviceWeight& w) { return w.view.type == T_Q4_K || w.view.type == T_Q5_K; };
       // attention block (gguf.cpp:1000-1060)
-      UAII_TRY(prep(pf_x_, d.dim, m, L.attn_norm, h16(L.wq) && h16(L.wk) && h16(L.wv)));
+      UAII_TRY(prep(pf_x_, d.dim, m, L.attn_norm, sums(L.wq) || sums(L.wk) || sums(L.wv)));
       const DeviceWeight* qkv[3] = {&L.wq, &L.wk, &L.wv};
       const int64_t qkv_cols[3] = {0, d.q_dim, d.q_dim + d.kv_dim};
       const int qkv_split = pf_store_split(qkv, 3, m, ldqkv);
@@ -811,14 +817,13 @@ Error DecoderProgram::prefill_rows(int64_t n) {
       UAII_TRY(timed("pf_attention", 4.0 * pairs * (double)d.kv_dim, 4.0 * pairs * (double)d.q_dim, [&] {
         return opts_.kv_f16 ? launch_pf_attn(at, s) : launch_pf_attn_f32(at, s);
       }));
-      UAII_TRY(prep(pf_attn_, d.q_dim, m, nullptr, h16(L.wo)));
+      UAII_TRY(prep(pf_attn_, d.q_dim, m, nullptr, sums(L.wo)));
       const DeviceWeight* wo[3] = {&L.wo, nullptr, nullptr};
       const int64_t c00[3] = {0, 0, 0};
       UAII_TRY(gemm("pf_gemm_o", wo, c00, 1, nullptr, EPI_ADD, m, pf_x_, d.dim));
       // FFN block (gguf.cpp:1130-1173)
       if (ls.ffn == LayerSpec::kSwiGLU || ls.ffn == LayerSpec::kGelu) {
-        const bool ffn16 = ls.ffn == LayerSpec::kSwiGLU ? h16(L.gate) && h16(L.up) : h16(L.up);
-        UAII_TRY(prep(pf_x_, d.dim, m, L.ffn_norm, ffn16));
+        UAII_TRY(prep(pf_x_, d.dim, m, L.ffn_norm, sums(L.up)));  // gate and up share a format
         if (ls.ffn == LayerSpec::kSwiGLU) {
           const DeviceWeight* wg[3] = {&L.gate, nullptr, nullptr};
           UAII_TRY(gemm("pf_gemm_gate_up", wg, c00, 1, &L.up, EPI_SWIGLU, m, pf_h_, ls.inter));
@@ -826,7 +831,7 @@ Error DecoderProgram::prefill_rows(int64_t n) {
           const DeviceWeight* wu[3] = {&L.up, nullptr, nullptr};
           UAII_TRY(gemm("pf_gemm_up", wu, c00, 1, nullptr, EPI_GELU, m, pf_h_, ls.inter));
         }
-        UAII_TRY(prep(pf_h_, ls.inter, m, nullptr, h16(L.down)));
+        UAII_TRY(prep(pf_h_, ls.inter, m, nullptr, sums(L.down)));
         const DeviceWeight* wd[3] = {&L.down, nullptr, nullptr};
         UAII_TRY(gemm("pf_gemm_down", wd, c00, 1, nullptr, EPI_ADD, m, pf_x_, d.dim));
       } else if (ls.ffn == LayerSpec::kMoE) {

@@ -153,7 +153,7 @@ class DecoderProgram {
   Error pf_gemm(const DeviceWeight* w[3], const int64_t cols0[3], int nw, const DeviceWeight* w2,
                 int epi, int64_t m, float* y, int64_t ldy, int store_split = 1);
   int pf_store_split(const DeviceWeight* w[3], int nw, int64_t m, int64_t ldy);
-  Error pf_prep(float* x, int64_t K, int64_t m, const float* norm_w, bool hi16 = false);
+  Error pf_prep(float* x, int64_t K, int64_t m, const float* norm_w, bool sums);
   template <class Prep, class Gemm>
   Error prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m, Prep&& prep, Gemm&& gemm);
   Error encode_step(bool want_logits);
@@ -175,7 +175,6 @@ class DecoderProgram {
   float* lm_part_val_ = nullptr;
   int32_t* lm_part_idx_ = nullptr;
   int lm_blocks_ = 0;  // capacity of the LM-head partial buffers
-  bool pf_h16_ = true;    // Q4_0 prefill GEMMs on PfAct::hi16 activations (UAII_PF_H16=0: off)
   // profiling mode: start/stop event pairs and their (kernel name, bytes) per launch group
   struct ProfTag {
     std::string name;
@@ -216,17 +215,17 @@ class DecoderProgram {
   bool moe_ = false;
 
   // prefill: chunk buffers ([chunk][...] rows) and the prepared-activation scratch
-  bool pf_ok_ = false;    // prefill(): the weights' formats and an f16 cache
+  bool pf_ok_ = false;    // prefill(): the weights' formats (pf_required) and an f16 cache
   bool pf_rows_ = false;  // generate_rows(): the weights' formats
   int64_t pf_chunk_ = 0, pf_kmax_ = 0;
   float *pf_x_ = nullptr, *pf_qkv_ = nullptr, *pf_q_ = nullptr, *pf_attn_ = nullptr,
         *pf_h_ = nullptr;
-  float* pf_part_ = nullptr;  // [4][chunk][dim]: K-split partials of a residual-add GEMM
+  float* pf_part_ = nullptr;  // K-split partials [split][rows][cols] of one GEMM
   // MoE prompt rows: routing [chunk][k], per-expert lists, expert outputs
   int32_t *pf_moe_ids_ = nullptr, *pf_moe_cnt_ = nullptr, *pf_moe_list_ = nullptr,
           *pf_moe_inv_ = nullptr, *pf_moe_tab_ = nullptr;
   int64_t pf_tab_cap_ = 0;             // int32 entries of pf_moe_tab_
-  int64_t pf_part_cols_ = 0;           // columns per row of pf_part_
+  int64_t pf_part_floats_ = 0;         // capacity of pf_part_
   std::vector<int32_t> pf_tab_host_;   // the grouped GEMMs' row tables before upload
   float *pf_moe_w_ = nullptr, *pf_moe_y_ = nullptr, *pf_hsh_ = nullptr;
   int pf_pending_ = 0;        // splits in pf_part_ still to be added into pf_x_
