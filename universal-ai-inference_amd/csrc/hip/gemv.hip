@@ -671,7 +671,7 @@ __device__ inline int epi_pos(const GemvArgs& a) {
   return 0;
 }
 
-template <int FMT, int EPI>
+template <int FMT, int EPI, int NJ = 2>
 __device__ inline void load_unit(const GemvArgs& a, const GemvSeg& seg, int64_t ebase, const Walk& wk,
                                  int64_t l0, int step, int lane, int pos, UnitBuf<FMT>& U) {
   constexpr int R = rpw_of(FMT);
@@ -683,7 +683,7 @@ __device__ inline void load_unit(const GemvArgs& a, const GemvSeg& seg, int64_t 
   // conservative at the join and serialise the unit's loads.)
   const int ncol = (int)((wk.nch + 63) / 64);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < NJ; ++j) {
     const int col = min(wk.cbeg + 2 * step + j, ncol - 1);
     const int64_t t = min((int64_t)col * 64 + lane, wk.nch - 1);
 #pragma unroll
@@ -692,11 +692,11 @@ __device__ inline void load_unit(const GemvArgs& a, const GemvSeg& seg, int64_t 
   epi_load<EPI, R>(a, seg, l0, lane, pos, U.e);
 }
 
-template <int FMT>
+template <int FMT, int NJ = 2>
 __device__ inline void compute_unit(const Walk& wk, int step, int lane, const float* xsm,
                                     const UnitBuf<FMT>& U, float* acc) {
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < NJ; ++j) {
     const int col = wk.cbeg + 2 * step + j;  // wave-uniform
     {
       const int64_t t0 = (int64_t)min(col, (int)((wk.nch + 63) / 64) - 1) * 64 + lane;
@@ -1097,7 +1097,7 @@ __device__ inline void epilogue(const GemvArgs& a, const GemvSeg& seg, int64_t l
 }
 
 // The whole kernel for one format (the dynamic LDS, xsm, holds the staged input).
-template <int FMT, int EPI, int W, bool RT>
+template <int FMT, int EPI, int W, bool RT, bool N1 = false>
 __device__ __forceinline__ void gemv_body(GemvArgs a, float* xsm) {
   __shared__ float red[2 * W];
   __shared__ float kred[2][W][RPW_MAX];
@@ -1189,14 +1189,16 @@ __device__ __forceinline__ void gemv_body(GemvArgs a, float* xsm) {
     // decode (gate/up 19.3 -> 17.9 us, LM head 61 -> 55 us, QKV unchanged;
     // 461 -> 471 tok/s).
     stage_pairs_finish<FMT, W * 64, RT>(a, xin, wk.nch, ps0, xsm, red);
-    if (nunits > 0) load_unit<FMT, EPI>(a, seg, ebase, wk, unit_l0(0), 0, lane, pos, U0);
+    if constexpr (!N1)
+      if (nunits > 0) load_unit<FMT, EPI>(a, seg, ebase, wk, unit_l0(0), 0, lane, pos, U0);
   } else if constexpr (FMT == T_Q8_0) {
     // input first here too: 8B Q8_0 decode 368.4 -> 372.2 tok/s (QKV 13.0 -> 12.0
     // us); the same order for the K-quants measured slower (1B 935 -> 917 tok/s)
     stage_x<FMT, W * 64, RT>(a, xin, wk.nch, xsm, red);
     if (nunits > 0) load_unit<FMT, EPI>(a, seg, ebase, wk, unit_l0(0), 0, lane, pos, U0);
   } else {
-    if (nunits > 0) load_unit<FMT, EPI>(a, seg, ebase, wk, unit_l0(0), 0, lane, pos, U0);
+    if constexpr (!N1)
+      if (nunits > 0) load_unit<FMT, EPI>(a, seg, ebase, wk, unit_l0(0), 0, lane, pos, U0);
     stage_x<FMT, W * 64, RT>(a, xin, wk.nch, xsm, red);
   }
 
@@ -1259,6 +1261,26 @@ __device__ __forceinline__ void gemv_body(GemvArgs a, float* xsm) {
 #pragma unroll
     for (int r = 0; r < RPW; ++r) acc[r] = 0.0f;
   };
+  // N1: rows of one chunk column (32-value chunks up to K = 2048). A unit's second
+  // column would load the first again and drop its dot, so two row groups share the
+  // batch instead, with the same loads in flight and each of them used. 128256 x 2048:
+  // Q6_K 72.0 -> 43.9 us, Q4_K 61.9 -> 42.6, Q4_0 51.1 -> 31.2; 2048 x 2048 Q6_K
+  // 5.3 -> 4.7; 1B decode 1391 -> 1491 tok/s. An instance of its own: as a branch beside
+  // the wide walk it cost that 6 % (8B gate/up 14.9 -> 15.8 us).
+  if constexpr (N1) {
+    for (int u = 0; u < nunits; u += 2) {
+      UnitBuf<FMT> V0, V1;
+      const int u1 = min(u + 1, nunits - 1);  // loaded again past the end, not finished
+      load_unit<FMT, EPI, 1>(a, seg, ebase, wk, unit_l0(u), 0, lane, pos, V0);
+      load_unit<FMT, EPI, 1>(a, seg, ebase, wk, unit_l0(u1), 0, lane, pos, V1);
+      compute_unit<FMT, 1>(wk, 0, lane, xs, V0, acc);
+      finish(u, V0.e);
+      if (u + 1 < nunits) {
+        compute_unit<FMT, 1>(wk, 0, lane, xs, V1, acc);
+        finish(u + 1, V1.e);
+      }
+    }
+  } else
   // first batch: unit 0 (already in flight) and, for NB = 2, unit 1
   if constexpr (NB == 1) {
     if (nunits > 0) {
@@ -1317,23 +1339,23 @@ __device__ __forceinline__ void gemv_body(GemvArgs a, float* xsm) {
 // took 130 VGPRs and held one block per CU; capped at 128 (2 spilled) the
 // Mixtral-shape QKV ran 12.8 -> 9.6 us. The two-format kernel keeps its 132:
 // capped, its 6 spills made the 1B QKV slower.
-template <int FMT, int EPI, int W, bool RT>
+template <int FMT, int EPI, int W, bool RT, bool N1 = false>
 __global__ void __launch_bounds__(W * 64, W == 8 ? 4 : 1) k_gemv(GemvArgs a) {
   extern __shared__ float xsm[];
-  gemv_body<FMT, EPI, W, RT>(a, xsm);
+  gemv_body<FMT, EPI, W, RT, N1>(a, xsm);
 }
 
 // Segments of two formats in one launch (a QKV whose V projection is stored in
 // another format, as in Q4_K_M files: Q4_K Q/K, Q6_K V). Blocks belong to one
 // segment, so each block stages and walks in its own segment's format; the
 // per-format launches this replaces each paid their own ramp and input staging.
-template <int FA, int FB, int EPI, int W, bool RT>
+template <int FA, int FB, int EPI, int W, bool RT, bool N1>
 __global__ void __launch_bounds__(W * 64) k_gemv_mix(GemvArgs a) {
   extern __shared__ float xsm[];
   int si = 0;
   for (int k = 1; k < a.nseg; ++k) if ((int)blockIdx.x >= a.seg[k].block0) si = k;
-  if (a.seg[si].w.type == FB) gemv_body<FB, EPI, W, RT>(a, xsm);
-  else gemv_body<FA, EPI, W, RT>(a, xsm);
+  if (a.seg[si].w.type == FB) gemv_body<FB, EPI, W, RT, N1>(a, xsm);
+  else gemv_body<FA, EPI, W, RT, N1>(a, xsm);
 }
 
 // Final greedy argmax over the LM-head block partials (lowest index wins ties,
@@ -1389,8 +1411,25 @@ __global__ void __launch_bounds__(1024) k_argmax_final(GemvArgs a, int nparts) {
 
 using KernelFn = void (*)(GemvArgs);
 
+// Formats whose rows of one chunk column (n1) take a walk of their own.
+bool narrow_fmt(int type) {
+  return type == T_Q4_0 || type == T_Q4_1 || type == T_Q4_K || type == T_Q5_K || type == T_Q6_K;
+}
+
 template <int EPI, int W, bool RT>
-KernelFn pick_fmt(int type) {
+KernelFn pick_fmt(int type, bool n1) {
+  if constexpr (EPI != EPI_ADD2 && W != WPB_LONG) {
+    if (n1) {
+      switch (type) {
+        case T_Q4_0: return k_gemv<T_Q4_0, EPI, W, RT, true>;
+        case T_Q4_1: return k_gemv<T_Q4_1, EPI, W, RT, true>;
+        case T_Q4_K: return k_gemv<T_Q4_K, EPI, W, RT, true>;
+        case T_Q5_K: return k_gemv<T_Q5_K, EPI, W, RT, true>;
+        case T_Q6_K: return k_gemv<T_Q6_K, EPI, W, RT, true>;
+        default: return nullptr;
+      }
+    }
+  }
   switch (type) {
     case T_Q4_0: return k_gemv<T_Q4_0, EPI, W, RT>;
     case T_Q8_0: return k_gemv<T_Q8_0, EPI, W, RT>;
@@ -1414,44 +1453,47 @@ KernelFn pick_fmt(int type) {
 // its own instances of the epilogues that take a residual as input: the copy in
 // the staging slowed every launch that carried it, taken or not (1B decode
 // 1220 -> 1193 tok/s).
-KernelFn pick(int epi, int type, int w, bool rt) {
+KernelFn pick(int epi, int type, int w, bool rt, bool n1) {
   if (rt) {
-    if (epi == EPI_SWIGLU && w == WPB_SWIGLU) return pick_fmt<EPI_SWIGLU, WPB_SWIGLU, true>(type);
-    if (epi == EPI_QKV && w == WPB_QKV) return pick_fmt<EPI_QKV, WPB_QKV, true>(type);
+    if (epi == EPI_SWIGLU && w == WPB_SWIGLU) return pick_fmt<EPI_SWIGLU, WPB_SWIGLU, true>(type, n1);
+    if (epi == EPI_QKV && w == WPB_QKV) return pick_fmt<EPI_QKV, WPB_QKV, true>(type, n1);
     if (w != WPB) return nullptr;
     switch (epi) {
-      case EPI_STORE: return pick_fmt<EPI_STORE, WPB, true>(type);
-      case EPI_QKV: return pick_fmt<EPI_QKV, WPB, true>(type);
-      case EPI_SWIGLU: return pick_fmt<EPI_SWIGLU, WPB, true>(type);
-      case EPI_LOGITS: return pick_fmt<EPI_LOGITS, WPB, true>(type);
-      case EPI_GELU: return pick_fmt<EPI_GELU, WPB, true>(type);
+      case EPI_STORE: return pick_fmt<EPI_STORE, WPB, true>(type, n1);
+      case EPI_QKV: return pick_fmt<EPI_QKV, WPB, true>(type, n1);
+      case EPI_SWIGLU: return pick_fmt<EPI_SWIGLU, WPB, true>(type, n1);
+      case EPI_LOGITS: return pick_fmt<EPI_LOGITS, WPB, true>(type, n1);
+      case EPI_GELU: return pick_fmt<EPI_GELU, WPB, true>(type, n1);
       default: return nullptr;
     }
   }
-  if (epi == EPI_SWIGLU && w == WPB_SWIGLU) return pick_fmt<EPI_SWIGLU, WPB_SWIGLU, false>(type);
-  if (epi == EPI_QKV && w == WPB_QKV) return pick_fmt<EPI_QKV, WPB_QKV, false>(type);
+  if (epi == EPI_SWIGLU && w == WPB_SWIGLU) return pick_fmt<EPI_SWIGLU, WPB_SWIGLU, false>(type, n1);
+  if (epi == EPI_QKV && w == WPB_QKV) return pick_fmt<EPI_QKV, WPB_QKV, false>(type, n1);
   if (w == WPB_LONG) {
-    if (epi == EPI_ADD) return pick_fmt<EPI_ADD, WPB_LONG, false>(type);
-    if (epi == EPI_ADD2) return pick_fmt<EPI_ADD2, WPB_LONG, false>(type);
+    if (epi == EPI_ADD) return pick_fmt<EPI_ADD, WPB_LONG, false>(type, n1);
+    if (epi == EPI_ADD2) return pick_fmt<EPI_ADD2, WPB_LONG, false>(type, n1);
     return nullptr;
   }
   if (w != WPB) return nullptr;
   switch (epi) {
-    case EPI_STORE: return pick_fmt<EPI_STORE, WPB, false>(type);
-    case EPI_ADD: return pick_fmt<EPI_ADD, WPB, false>(type);
-    case EPI_QKV: return pick_fmt<EPI_QKV, WPB, false>(type);
-    case EPI_SWIGLU: return pick_fmt<EPI_SWIGLU, WPB, false>(type);
-    case EPI_LOGITS: return pick_fmt<EPI_LOGITS, WPB, false>(type);
-    case EPI_GELU: return pick_fmt<EPI_GELU, WPB, false>(type);
+    case EPI_STORE: return pick_fmt<EPI_STORE, WPB, false>(type, n1);
+    case EPI_ADD: return pick_fmt<EPI_ADD, WPB, false>(type, n1);
+    case EPI_QKV: return pick_fmt<EPI_QKV, WPB, false>(type, n1);
+    case EPI_SWIGLU: return pick_fmt<EPI_SWIGLU, WPB, false>(type, n1);
+    case EPI_LOGITS: return pick_fmt<EPI_LOGITS, WPB, false>(type, n1);
+    case EPI_GELU: return pick_fmt<EPI_GELU, WPB, false>(type, n1);
     default: return nullptr;
   }
 }
 
 // The two-format kernel: QKV with Q4_K and Q6_K segments.
-KernelFn pick_mix(int epi, int w, bool rt) {
-  if (epi == EPI_QKV && w == WPB_QKV)
-    return rt ? k_gemv_mix<T_Q4_K, T_Q6_K, EPI_QKV, WPB_QKV, true> : k_gemv_mix<T_Q4_K, T_Q6_K, EPI_QKV, WPB_QKV, false>;
-  return nullptr;
+KernelFn pick_mix(int epi, int w, bool rt, bool n1) {
+  if (epi != EPI_QKV || w != WPB_QKV) return nullptr;
+  if (n1)
+    return rt ? k_gemv_mix<T_Q4_K, T_Q6_K, EPI_QKV, WPB_QKV, true, true>
+              : k_gemv_mix<T_Q4_K, T_Q6_K, EPI_QKV, WPB_QKV, false, true>;
+  return rt ? k_gemv_mix<T_Q4_K, T_Q6_K, EPI_QKV, WPB_QKV, true, false>
+            : k_gemv_mix<T_Q4_K, T_Q6_K, EPI_QKV, WPB_QKV, false, false>;
 }
 
 // Waves per block for a launch of epilogue `epi` whose rows split K over `ks` waves.
@@ -1474,14 +1516,15 @@ hipError_t prepare_gemv() {
   const int lim = lds_limit();
   for (int e : epis) {
     for (int w : {WPB, WPB_QKV, WPB_SWIGLU, WPB_LONG}) {
-      for (bool rt : {false, true}) {
+      for (int v = 0; v < 4; ++v) {
+        const bool rt = v & 1, n1 = v & 2;
         for (int t : types) {
-          const KernelFn fn = pick(e, t, w, rt);
+          const KernelFn fn = n1 && !narrow_fmt(t) ? nullptr : pick(e, t, w, rt, n1);
           if (!fn) continue;
           (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lim - 1024);
           (void)hipGetLastError();
         }
-        if (const KernelFn fn = pick_mix(e, w, rt)) {
+        if (const KernelFn fn = pick_mix(e, w, rt, n1)) {
           (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lim - 1024);
           (void)hipGetLastError();
         }
@@ -1568,7 +1611,12 @@ Plan make_plan(const GemvArgs& a) {
   p.ks = pick_ksplit(a.seg[0].w);
   p.waves = pick_waves(a.epi, p.ks);
   const bool rt = a.rtap != nullptr;
-  p.fn = mix ? pick_mix(a.epi, p.waves, rt) : pick(a.epi, a.seg[0].w.type, p.waves, rt);
+  // Rows of one 64-chunk column, up to 2048 values in these formats, take the two-group
+  // walk at every row count: 512 x 1024 Q4_0 5.3 -> 4.7 us, 128256 x 2048 51.1 -> 31.2.
+  // From 2080 values on a unit's second column is real work and the wide walk holds.
+  bool n1 = !pair;
+  for (int k = 0; k < a.nseg; ++k) n1 = n1 && a.seg[k].w.a_row <= 1024 && narrow_fmt(a.seg[k].w.type);
+  p.fn = mix ? pick_mix(a.epi, p.waves, rt, n1) : pick(a.epi, a.seg[0].w.type, p.waves, rt, n1);
   if (!p.fn) return p;
   const int rpg = (p.waves / (pair ? 2 : 1) / p.ks) * rpw_of(a.seg[0].w.type);
   if (pair) {
