@@ -206,33 +206,62 @@ constexpr int PA_TK = 64;  // keys per LDS tile
 #endif
 constexpr int PA_QW = UAII_PA_QW;
 
-// Block: 4 waves on kv head blockIdx.y / (G / GW); wave w takes q head
+// Four f16 of the transposed 4 x 16 piece that a group of 16 lanes names (8 bytes each).
+__device__ inline h4_t lds_tr4(const _Float16* p) {
+  typedef short s4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s4_t* lds4;
+  return __builtin_bit_cast(h4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p));
+}
+
+// Query tile of the xi-th of nx tiles in launch order: the longest first, and every
+// other band (the tiles of one block a CU) the other way round.
+__device__ inline int pf_attn_tile(int xi, int nx, int band) {
+  const int b = xi / band;
+  if (b & 1) xi = b * band + min(band, nx - b * band) - 1 - (xi - b * band);
+  return nx - 1 - xi;
+}
+
+// Block: 4 waves on kv head hb / (G / GW); wave w takes q head
 // (w % GW) of the block's GW heads and query subtiles PA_QW (w / GW) ..
-// PA_QW (w / GW) + PA_QW - 1 (16 queries each). K tiles and transposed V tiles
-// of 64 keys are double-buffered in LDS; each thread loads the next tile's K/V
+// PA_QW (w / GW) + PA_QW - 1 (16 queries each). K and V tiles of 64 keys are
+// double-buffered in LDS as they lie in the cache; each thread loads the next tile's
 // pieces into registers while the current tile is computed.
+//
+// What bounds it: the softmax between the two products of a wave's tile (two waves a
+// SIMD cover each other), with the hi/lo products at twice the plain matrix-core work.
+// V was stored transposed, 4 bytes a lane with rows 288 words apart: 8 lanes to a bank
+// on every store, as much LDS time as all fragment reads together, and 16 vector
+// operations a piece to pair the keys. Stored plain and read by ds_read_b64_tr_b16
+// (two conflict-free reads a fragment, as before), with the probabilities' hi and lo
+// halves one fused operation each: 1024 queries at 1024, 32/8 heads of 128,
+// 139 -> 80 us between calls from the host, 138 -> 66 back to back with the band order
+// below (25.8 GFLOP: 187 -> 391 TFLOP/s); 512 queries at 4096 210 -> 125 us, where one
+// block a CU leaves the softmax uncovered; 1000 from 0 at head_dim 64 36 -> 24 us.
+// Blocks are numbered head first, so that an XCD's blocks share the K/V of few heads in
+// its L2, with the longest query tiles first and alternate bands reversed, which gives
+// the two blocks of a CU a long and a short tile: 79.8 -> 77.6 us, 2048 from 0
+// 98.2 -> 94.9 us.
 template <int HD>
 __global__ void __launch_bounds__(256, 2) k_pf_attn(PfAttnArgs a) {
   constexpr int KP = HD + 8;        // K tile row (halfs)
-  constexpr int VP = PA_TK + 8;     // V^T tile row (halfs)
   constexpr int NC = HD / 32;       // 32-wide hd chunks (S)
   constexpr int ND = HD / 16;       // 16-row hd subtiles (O)
-  constexpr int KPIECES = PA_TK * (HD / 8) / 256;       // 16-byte K pieces per thread
-  constexpr int VPAIRS = PA_TK / 2 * (HD / 8) / 256;    // (2 keys x 8 dims) V pieces per thread
+  constexpr int PIECES = PA_TK * (HD / 8) / 256;  // 16-byte K (and V) pieces per thread
   __shared__ _Float16 ks[2][PA_TK * KP];
-  __shared__ _Float16 vt[2][HD * VP];
+  __shared__ _Float16 vs[2][PA_TK * KP];
 
   const int G = a.n_heads / a.n_kv;
   const int GW = G < 4 ? G : 4;
   const int QS = 4 / GW;
-  const int hb = blockIdx.y;
+  const int ny = a.n_kv * (G / GW);
+  const int hb = (int)blockIdx.x % ny;
   const int kvh = hb / (G / GW);
   const int hbase = kvh * G + (hb % (G / GW)) * GW;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const bool active = wave < GW * QS;
   const int head = hbase + (wave % GW);
-  const int64_t q0 = (int64_t)blockIdx.x * (16 * PA_QW * QS);
+  const int64_t q0 = (int64_t)pf_attn_tile((int)blockIdx.x / ny, (int)gridDim.x / ny, a.band) * (16 * PA_QW * QS);
   const int64_t qw0 = q0 + 16 * PA_QW * (wave / GW);   // this wave's first query
   const int64_t qend = min((int64_t)a.M, q0 + 16 * PA_QW * QS);
   const int64_t nkeys = a.p0 + qend;  // keys the block needs (causal)
@@ -313,51 +342,30 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn(PfAttnArgs a) {
   // tile staging: K pieces (key, 8 dims) and V pairs (keys 2k, 2k + 1, 8 dims);
   // keys past nkeys read as zeros. Offsets inside a tile are 32-bit and fixed
   // per thread; only the last tile checks them against nkeys.
-  uint4 kreg[KPIECES], vreg[VPAIRS][2];
+  uint4 kreg[PIECES], vreg[PIECES];
   auto load_tile = [&](int64_t kt) __attribute__((always_inline)) {
     const __half* kt_base = reinterpret_cast<const __half*>(uniform_ptr(kbase + kt * HD));
     const __half* vt_base = reinterpret_cast<const __half*>(uniform_ptr(vbase + kt * HD));
     const bool full = kt + PA_TK <= nkeys;  // block-uniform
 #pragma unroll
-    for (int u = 0; u < KPIECES; ++u) {
+    for (int u = 0; u < PIECES; ++u) {
       const int c = threadIdx.x + 256 * u;
       const int key = c / (HD / 8), p = c % (HD / 8);
       kreg[u] = make_uint4(0, 0, 0, 0);
-      if (full || kt + key < nkeys) kreg[u] = *reinterpret_cast<const uint4*>(kt_base + (key * HD + 8 * p));
-    }
-#pragma unroll
-    for (int u = 0; u < VPAIRS; ++u) {
-      const int c = threadIdx.x + 256 * u;
-      const int kp = c / (HD / 8), p = c % (HD / 8);
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        vreg[u][e] = make_uint4(0, 0, 0, 0);
-        if (full || kt + 2 * kp + e < nkeys)
-          vreg[u][e] = *reinterpret_cast<const uint4*>(vt_base + ((2 * kp + e) * HD + 8 * p));
+      vreg[u] = make_uint4(0, 0, 0, 0);
+      if (full || kt + key < nkeys) {
+        kreg[u] = *reinterpret_cast<const uint4*>(kt_base + (key * HD + 8 * p));
+        vreg[u] = *reinterpret_cast<const uint4*>(vt_base + (key * HD + 8 * p));
       }
     }
   };
   auto store_tile = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < KPIECES; ++u) {
+    for (int u = 0; u < PIECES; ++u) {
       const int c = threadIdx.x + 256 * u;
       const int key = c / (HD / 8), p = c % (HD / 8);
       *reinterpret_cast<uint4*>(&ks[buf][key * KP + 8 * p]) = kreg[u];
-    }
-#pragma unroll
-    for (int u = 0; u < VPAIRS; ++u) {
-      const int c = threadIdx.x + 256 * u;
-      const int kp = c / (HD / 8), p = c % (HD / 8);
-      const uint32_t w0[4] = {vreg[u][0].x, vreg[u][0].y, vreg[u][0].z, vreg[u][0].w};
-      const uint32_t w1[4] = {vreg[u][1].x, vreg[u][1].y, vreg[u][1].z, vreg[u][1].w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        // dims 8p + 2e and 8p + 2e + 1 of keys 2kp and 2kp + 1, as key pairs
-        const uint32_t lo = (w0[e] & 0xffffu) | (w1[e] << 16);
-        const uint32_t hi = (w0[e] >> 16) | (w1[e] & 0xffff0000u);
-        *reinterpret_cast<uint32_t*>(&vt[buf][(8 * p + 2 * e) * VP + 2 * kp]) = lo;
-        *reinterpret_cast<uint32_t*>(&vt[buf][(8 * p + 2 * e + 1) * VP + 2 * kp]) = hi;
-      }
+      *reinterpret_cast<uint4*>(&vs[buf][key * KP + 8 * p]) = vreg[u];
     }
   };
   auto lds_barrier = []() __attribute__((always_inline)) {
@@ -428,20 +436,24 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn(PfAttnArgs a) {
         h8_t phi, plo;
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
-          const float p = sc[2 * c + (r >> 2)][r & 3] * 16384.0f;
-          const _Float16 h = (_Float16)p;
+          const float p = sc[2 * c + (r >> 2)][r & 3];
+          const _Float16 h = (_Float16)(p * 16384.0f);
           phi[r] = h;
-          plo[r] = (_Float16)(p - (float)h);
+          plo[r] = (_Float16)fmaf(p, 16384.0f, -(float)h);  // exact before the rounding
         }
+        // V^T by transposed LDS reads: the 16 lanes of group g name 4 keys x 16 dims,
+        // lane i gets dim i of the 4 keys
+        h8_t vf[ND];
 #pragma unroll
         for (int d = 0; d < ND; ++d) {
-          const _Float16* vr = &vt[buf][(16 * d + col) * VP + 32 * c + 4 * g];
-          const h4_t v0 = *reinterpret_cast<const h4_t*>(vr);
-          const h4_t v1 = *reinterpret_cast<const h4_t*>(vr + 16);
-          const h8_t vf = h8_t{v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-          o[u][d] = mfma32(vf, phi, o[u][d]);
-          o[u][d] = mfma32(vf, plo, o[u][d]);
+          const _Float16* vr = &vs[buf][(32 * c + 4 * g + (col >> 2)) * KP + 16 * d + 4 * (col & 3)];
+          const h4_t v0 = lds_tr4(vr), v1 = lds_tr4(vr + 16 * KP);
+          vf[d] = h8_t{v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
         }
+#pragma unroll
+        for (int d = 0; d < ND; ++d) o[u][d] = mfma32(vf[d], phi, o[u][d]);
+#pragma unroll
+        for (int d = 0; d < ND; ++d) o[u][d] = mfma32(vf[d], plo, o[u][d]);
       }
     }
   };
@@ -820,9 +832,14 @@ hipError_t launch_pf_attn(const PfAttnArgs& a, hipStream_t s) {
   const int GW = G < 4 ? G : 4;
   const int QS = 4 / GW;
   const int QT = 16 * PA_QW * QS;  // queries per block
-  dim3 grid((unsigned)((a.M + QT - 1) / QT), (unsigned)(a.n_kv * (G / GW)));
-  if (a.hd == 64) UAII_LAUNCH(k_pf_attn<64>, grid, dim3(256), 0, s, a);
-  else UAII_LAUNCH(k_pf_attn<128>, grid, dim3(256), 0, s, a);
+  const int ny = a.n_kv * (G / GW);
+  const int64_t blocks = (int64_t)((a.M + QT - 1) / QT) * ny;
+  if (blocks > INT32_MAX) return hipErrorInvalidValue;
+  PfAttnArgs b = a;
+  b.band = std::max(1, device_cus() / ny);  // query tiles that give every CU one block
+  const dim3 grid((unsigned)blocks);
+  if (a.hd == 64) UAII_LAUNCH(k_pf_attn<64>, grid, dim3(256), 0, s, b);
+  else UAII_LAUNCH(k_pf_attn<128>, grid, dim3(256), 0, s, b);
   return hipGetLastError();
 }
 

@@ -327,6 +327,7 @@ struct PfAttnArgs {
   int64_t p0, M;        // queries at positions p0 .. p0 + M - 1 (keys 0 .. p0 + M - 1)
   float* out;           // [M][ldo]
   int64_t ldo;
+  int band;             // set by launch_pf_attn
 };
 
 // MoE prompt rows (transformer.cpp:446-612 applied to M tokens):
