@@ -1636,8 +1636,8 @@ Plan make_plan(const GemvArgs& a) {
   // CU measured 61.4 us against 65.0 with the argmax epilogue (1: 95.6, 2: 67.7,
   // 4: 64.1), 55.0 against 56.5 storing the logits for the device sampler;
   // 101.9 against 107.3 for the 558 MB Q8_0 head. Smaller heads keep every
-  // resident block: 70.7 against 76.7 us for a 148 MB Q4_K head (2048 columns),
-  // 28.7 against 29.4 for a 74 MB one.
+  // resident block: 70.7 against 76.7 us for a 148 MB Q4_K head (2048 columns, before
+  // its rows had a walk of their own; 42.6 us with it), 28.7 against 29.4 for a 74 MB one.
   const DevWeight& w0 = a.seg[0].w;
   const int64_t head_bytes = w0.rows * (w0.a_row + w0.b_row + w0.c_row + w0.d_row);
   const bool lm_head = a.epi == EPI_LOGITS || (a.epi == EPI_STORE && a.nseg == 1 && a.seg[0].rows >= 65536);

@@ -6,7 +6,9 @@
 // on v_mfma_f32_16x16x4_f32, whose products and sums are f32 as the token step's
 // are. That instruction does 64 multiply-adds' worth of flops per cycle and SIMD
 // (157 TFLOP/s dense, a sixteenth of the f16 rate), which is still far ahead of
-// what bounds a prompt: its GEMMs.
+// what bounds a prompt: its GEMMs. 1000 positions from 0, 32/8 heads of 64: 87 us a
+// layer, where token steps over the f32 cache took 1000 x 0.69 ms for all 16 layers
+// (whole run of 1000 + 8 ids 691 -> 14.4 ms).
 //
 // Operands of 16x16x4: lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16],
 // D[4 (l / 16) + r][l % 16] sits in element r. With S^T = K . Q^T the lane then
