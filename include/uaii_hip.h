@@ -90,7 +90,13 @@ UAII_HIP_API int uaii_hip_gemv_swiglu(const uaii_hip_weight* wg, const uaii_hip_
  * (weights decoded to their exact small integers, x split into f16 hi + lo, block
  * scales applied to the f32 sums); other formats run one GEMV per row. Q4_0 and Q8_0 need m (rounded up to 64)
  * * cols * 2 < 2^31 (their kernels address the f16 activation rows by 32-bit
- * byte offsets); larger calls return hipErrorInvalidValue. */
+ * byte offsets); larger calls return hipErrorInvalidValue.
+ * Scratch: the matrix-core calls and the decode attentions that allocate keep what they
+ * need between launches in device memory the library owns, grown on demand (which may
+ * wait for earlier calls of the same stream) and kept until the process ends. Calls on
+ * different streams and threads are independent. Calls captured into graphs share one
+ * buffer per GPU: order the replays of graphs that hold them, and a capture's branches;
+ * Q5_K and F16 calls are captured as one GEMV per row and need none. */
 UAII_HIP_API int uaii_hip_gemm(const uaii_hip_weight* w, const float* x, int64_t m, float* y,
                                void* stream);
 UAII_HIP_API int uaii_hip_gemm_rmsnorm(const uaii_hip_weight* w, const float* x, int64_t m,
@@ -148,10 +154,8 @@ UAII_HIP_API int uaii_hip_rope_table(float theta, int head_dim, int64_t max_pos,
 UAII_HIP_API int uaii_hip_rope(float* x, int64_t rows, int64_t dim, int head_dim, int mode,
                                const int32_t* pos_dev, const float* table_dev, void* stream);
 /* kcache/vcache: head-major [n_kv_heads][max_seq][head_dim], f16 (kv_f16=1) or f32;
- * attends over keys 0..n_keys-1. The split partials go to one device buffer the
- * library owns (grown on demand, kept until the process ends; growing it waits
- * for the device), shared with uaii_hip_attention_o: calls that run at the same
- * time on different streams race on it, so issue them on one stream. */
+ * attends over keys 0..n_keys-1. The split partials go to the library's scratch
+ * (see uaii_hip_gemm). */
 UAII_HIP_API int uaii_hip_attention_decode(const float* q, const void* kcache,
                                            const void* vcache, int kv_f16, int64_t max_seq,
                                            int n_heads, int n_kv_heads, int head_dim,
@@ -176,8 +180,8 @@ UAII_HIP_API int uaii_hip_gemv_add_atomic(const uaii_hip_weight* w, const float*
  * Q8_0 or Q4_K, [rows][n_heads * head_dim] with n_heads * head_dim a multiple of 256,
  * head_dim 64 or 128, rows (y's length) a multiple of 32; other shapes return
  * -1 and launch nothing, as do `out` and y overlapping (merge blocks write
- * `out` while others add into y). Its split partials share uaii_hip_attention_decode's
- * library-owned buffer (the same one-stream rule applies). */
+ * `out` while others add into y). Its split partials go to the library's scratch
+ * (see uaii_hip_gemm). */
 UAII_HIP_API int uaii_hip_attention_o(const float* q, const void* kcache, const void* vcache,
                                       int kv_f16, int64_t max_seq, int n_heads,
                                       int n_kv_heads, int head_dim, int64_t n_keys,

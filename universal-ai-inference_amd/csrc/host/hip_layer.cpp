@@ -2,9 +2,10 @@
 #include "uaii_hip.h"
 
 #include "program.h"
+#include "scratch.h"
 
 #include <cmath>
-#include <mutex>
+#include <optional>
 #include <random>
 #include <vector>
 
@@ -20,28 +21,7 @@ constexpr int kErrArg = -1;      // invalid argument
 constexpr int kErrNotImpl = -2;  // not implemented
 constexpr int kErrScratch = -3;  // larger than the allocation-free scratch
 
-std::mutex g_scratch_mu;
-void* g_scratch = nullptr;       // attention partials for uaii_hip_attention_decode
-size_t g_scratch_bytes = 0;
-
 hipStream_t S(void* s) { return static_cast<hipStream_t>(s); }
-
-int grow_scratch(size_t bytes) {
-  if (bytes <= g_scratch_bytes) return 0;
-  if (g_scratch) {
-    hipError_t e = hipDeviceSynchronize();
-    if (e != hipSuccess) return (int)e;
-    (void)hipFree(g_scratch);
-    g_scratch = nullptr;
-    g_scratch_bytes = 0;
-  }
-  hipError_t e = hipMalloc(&g_scratch, bytes);
-  if (e != hipSuccess) return (int)e;
-  e = hipMemset(g_scratch, 0, bytes);
-  if (e != hipSuccess) return (int)e;
-  g_scratch_bytes = bytes;
-  return 0;
-}
 
 }  // namespace
 
@@ -168,7 +148,7 @@ int uaii_hip_gemv_swiglu(const uaii_hip_weight* wg, const uaii_hip_weight* wu, c
 namespace {
 
 // M-row products: the MFMA kernel for the block formats it decodes, else one
-// GEMV launch per row (same epilogue). Prepared activations live in g_scratch.
+// GEMV launch per row (same epilogue). Prepared activations live in a Scratch.
 int gemm_common(const uaii_hip_weight* w, const uaii_hip_weight* w2, const float* x, int64_t m,
                 const float* norm_w, float eps, float* y, int epi, void* stream) {
   if (!w || !x || !y || m <= 0) return kErrArg;
@@ -195,7 +175,12 @@ int gemm_common(const uaii_hip_weight* w, const uaii_hip_weight* w2, const float
   const bool required = pf_required(v.type);
   if (!pf_supported(v.type) || K % 64) return row_by_row();
   if (!required && (!pf_row_supported(K) || m > 65535 * 64)) return row_by_row();
-  std::unique_lock<std::mutex> lk(g_scratch_mu);
+  std::optional<uaii::Scratch> scratch(std::in_place, S(stream));
+  // A graph of row-by-row calls holds the caller's pointers only, and its replays may overlap.
+  if (!required && scratch->capturing()) {
+    scratch.reset();
+    return row_by_row();
+  }
   const int64_t mpad = pf_mpad(m);
   PfGemmArgs a{};
   a.nseg = 1;
@@ -214,30 +199,23 @@ int gemm_common(const uaii_hip_weight* w, const uaii_hip_weight* w2, const float
   a.ksplit = pf_gemm_ksplit(a, pf_device_cus(), (int64_t)16 << 20);
   a.ldp = epi == EPI_SWIGLU ? 2 * N : N;
   const size_t hb = (size_t)mpad * (size_t)K * 2, xb = K % 256 == 0 ? hb / 8 : 0, rb = (size_t)mpad * 4;
-  auto reserve = [&]() -> int {
+  auto reserve = [&]() -> hipError_t {
     const size_t pb = a.ksplit > 1 ? (size_t)a.ksplit * (size_t)m * (size_t)a.ldp * 4 : 0;
-    const size_t need = 2 * hb + xb + rb + pb;
-    if (need <= g_scratch_bytes) return 0;
-    // growing allocates, which a captured stream does not allow
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (stream && (a.ksplit > 1 || !required) && hipStreamIsCapturing(S(stream), &cs) == hipSuccess &&
-        cs != hipStreamCaptureStatusNone)
-      return (int)hipErrorStreamCaptureUnsupported;
-    return grow_scratch(need);
+    return scratch->reserve(2 * hb + xb + rb + pb);
   };
-  int rc = reserve();
-  if (rc && a.ksplit > 1) {
+  hipError_t e = reserve();
+  if (e != hipSuccess && a.ksplit > 1) {
     (void)hipGetLastError();
     a.ksplit = 1;
-    rc = reserve();
+    e = reserve();
   }
-  if (rc && !required) {
+  if (e != hipSuccess && !required) {
     (void)hipGetLastError();
-    lk.unlock();
+    scratch.reset();
     return row_by_row();
   }
-  if (rc) return rc;
-  char* base = static_cast<char*>(g_scratch);
+  if (e != hipSuccess) return (int)e;
+  char* base = scratch->data();
   PfAct act{};
   act.hi = reinterpret_cast<__half*>(base);
   act.lo = reinterpret_cast<__half*>(base + hb);
@@ -245,7 +223,7 @@ int gemm_common(const uaii_hip_weight* w, const uaii_hip_weight* w2, const float
   act.rs = reinterpret_cast<float*>(base + 2 * hb + xb);
   act.mpad = mpad;
   act.K = K;
-  hipError_t e = launch_pf_prep(const_cast<float*>(x), K, m, norm_w, eps, act, S(stream));
+  e = launch_pf_prep(const_cast<float*>(x), K, m, norm_w, eps, act, S(stream));
   if (e != hipSuccess) return (int)e;
   a.ahi = act.hi;
   a.alo = act.lo;
@@ -417,12 +395,12 @@ int uaii_hip_attention_decode(const float* q, const void* kcache, const void* vc
       n_heads % n_kv_heads || head_dim <= 0 || n_keys <= 0 || n_keys > max_seq ||
       max_seq > INT32_MAX)  // key positions are 32-bit in the kernels
     return kErrArg;
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
   const int splits = uaii_hip::attention_splits(max_seq);
   const int G = n_heads / n_kv_heads;
   const size_t part = (size_t)n_kv_heads * splits * G * (size_t)(head_dim + 2) * 4;
-  int rc = grow_scratch(part);
-  if (rc) return rc;
+  uaii::Scratch scratch(S(stream));
+  const hipError_t rs = scratch.reserve(part);
+  if (rs != hipSuccess) return (int)rs;
   AttnArgs a{};
   a.q = q;
   a.kcache = kcache;
@@ -435,7 +413,7 @@ int uaii_hip_attention_decode(const float* q, const void* kcache, const void* vc
   a.state = nullptr;
   a.fixed_len = (int)n_keys;
   a.out = out;
-  a.part = static_cast<float*>(g_scratch);
+  a.part = reinterpret_cast<float*>(scratch.data());
   a.splits = splits;
   return (int)launch_attention_decode(a, S(stream));
 }
@@ -465,7 +443,6 @@ int uaii_hip_attention_o(const float* q, const void* kcache, const void* vcache,
       n_heads % n_kv_heads || head_dim <= 0 || n_keys <= 0 || n_keys > max_seq ||
       max_seq > INT32_MAX)
     return kErrArg;
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
   const int splits = uaii_hip::attention_splits(max_seq);
   const int G = n_heads / n_kv_heads;
   MergeOArgs m{};
@@ -493,9 +470,10 @@ int uaii_hip_attention_o(const float* q, const void* kcache, const void* vcache,
     if (o0 < y1 && y0 < o1) return kErrArg;
   }
   const size_t part = (size_t)n_kv_heads * splits * G * (size_t)(head_dim + 2) * 4;
-  int rc = grow_scratch(part);
-  if (rc) return rc;
-  a.part = static_cast<float*>(g_scratch);
+  uaii::Scratch scratch(S(stream));
+  const hipError_t rs = scratch.reserve(part);
+  if (rs != hipSuccess) return (int)rs;
+  a.part = reinterpret_cast<float*>(scratch.data());
   const hipError_t st = launch_attention_splits(a, S(stream));
   if (st != hipSuccess) return (int)st;
   return (int)launch_merge_o(m, S(stream));
