@@ -40,15 +40,8 @@ __global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t l
   uint2* lo2 = reinterpret_cast<uint2*>(act.lo);
   // float4 i of the row: quad i % 8 of 32-block i / 8, in the order 0, 4, 1, 5, ...
   auto at = [&](int i) -> int64_t { return ((int64_t)(i >> 3) * act.mpad + t) * 8 + 2 * (i & 3) + ((i >> 2) & 1); };
-  float4* raw4 = reinterpret_cast<float4*>(act.raw);
-  auto raw_at = [&](int i) -> int64_t {
-    return (((int64_t)((i >> 2) & 1) * (K / 32) + (i >> 3)) * act.mpad + t) * 4 + (i & 3);
-  };
   if (t >= M) {
-    for (int i = tid; i < nv; i += NT) {
-      if (act.hi) hi2[at(i)] = lo2[at(i)] = make_uint2(0, 0);
-      if (act.raw) raw4[raw_at(i)] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
+    for (int i = tid; i < nv; i += NT) { hi2[at(i)] = make_uint2(0, 0); lo2[at(i)] = make_uint2(0, 0); }
     if (act.sxp) {
       for (int i = tid; i < nv / 8; i += NT)
         reinterpret_cast<uint2*>(act.sxp)[((int64_t)(i >> 3) * act.mpad + t) * 8 + (i & 7)] = make_uint2(0, 0);
@@ -62,10 +55,12 @@ __global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t l
   for (int i = tid; i < nv; i += NT) {
     float4 v = x4[i];
     if (nsplit > 0) {
-      // residual add of a K-split GEMM's partials
-      const f4_t p = split_sum<f4_t>(nsplit, [&](int z) {
-        return reinterpret_cast<const f4_t*>(part + ((int64_t)z * M + t) * ldx)[i];
-      });
+      // residual add of a K-split GEMM's partials, in split order
+      float4 p = reinterpret_cast<const float4*>(part + t * ldx)[i];
+      for (int z = 1; z < nsplit; ++z) {
+        const float4 q = reinterpret_cast<const float4*>(part + ((int64_t)z * M + t) * ldx)[i];
+        p.x += q.x; p.y += q.y; p.z += q.z; p.w += q.w;
+      }
       v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
       x4[i] = v;
     }
@@ -96,22 +91,17 @@ __global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t l
     }
     __syncthreads();  // red[] is reused below
   }
-  if (act.raw) {
-    for (int i = tid; i < nv; i += NT) raw4[raw_at(i)] = r4[i];
-    if (!act.hi) return;
-  }
   amax = wave_max(amax);
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < NT / 64; ++w) amax = fmaxf(amax, red[w]);
   // scale so that max |x| * 2^e lies in [2^14, 2^15): hi keeps 11 bits of every
-  // element near the top of the row and lo the next 11. The limits are where 2^e and
-  // 2^-e are normal numbers and the largest finite row still fits f16.
+  // element near the top of the row and lo the next 11
   int e = 0;
   if (amax > 0.0f) {
     const int ex = (int)((__float_as_uint(amax) >> 23) & 0xff) - 126;  // amax in [2^(ex-1), 2^ex)
-    e = min(126, max(-113, 15 - ex));
+    e = min(100, max(-100, 15 - ex));
   }
   const float s = pow2f_i(e);
   if (tid == 0) act.rs[t] = pow2f_i(-e);
@@ -122,9 +112,8 @@ __global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t l
       const float4 v = r4[i];
       const float y0 = v.x * s, y1 = v.y * s, y2 = v.z * s, y3 = v.w * s;
       const _Float16 h0 = (_Float16)y0, h1 = (_Float16)y1, h2 = (_Float16)y2, h3 = (_Float16)y3;
-      // an infinity is all in hi
-      auto rest = [](float y, _Float16 h) { return (_Float16)(fabsf(y) == INFINITY ? 0.0f : y - (float)h); };
-      const _Float16 l0 = rest(y0, h0), l1 = rest(y1, h1), l2 = rest(y2, h2), l3 = rest(y3, h3);
+      const _Float16 l0 = (_Float16)(y0 - (float)h0), l1 = (_Float16)(y1 - (float)h1);
+      const _Float16 l2 = (_Float16)(y2 - (float)h2), l3 = (_Float16)(y3 - (float)h3);
       // stored order (k0, k2, k1, k3)
       hi2[at(i)] = make_uint2(__builtin_bit_cast(uint32_t, h2_t{h0, h2}),
                           __builtin_bit_cast(uint32_t, h2_t{h1, h3}));
@@ -160,9 +149,12 @@ __global__ void __launch_bounds__(256) k_pf_qkv(PfQkvArgs a) {
   const int pos = a.p0 + (int)t;
   const float* row = a.qkv + t * a.ldq;
   // value x of this row: the GEMM's output, or the sum of its K-split partials
+  // in split order
   auto val = [&](int x) -> float {
     if (a.nsplit <= 1) return row[x];
-    return split_sum<float>(a.nsplit, [&](int z) { return a.part[((int64_t)z * a.M + t) * a.ldq + x]; });
+    float v = a.part[t * a.ldq + x];
+    for (int z = 1; z < a.nsplit; ++z) v = v + a.part[((int64_t)z * a.M + t) * a.ldq + x];
+    return v;
   };
   const int hd = a.head_dim, half = hd / 2;
   const int npair = (a.q_dim + a.kv_dim) / 2;
