@@ -88,7 +88,7 @@ UAII_HIP_API int uaii_hip_gemv_swiglu(const uaii_hip_weight* wg, const uaii_hip_
 /* M > 1: y[i][:] = W . x[i][:] for i < m (x [m][cols], y [m][rows]). Q4_0, Q8_0,
  * Q4_K, Q5_K, Q6_K and F16 with cols a multiple of 64 run on the matrix cores
  * (weights decoded to their exact small integers, x split into f16 hi + lo, block
- * scales applied to the f32 sums); other formats run one GEMV per row. Q4_0 and Q8_0 need m (rounded up to 64)
+ * scales applied to the f32 sums; F16 weights and x as f32); other formats run one GEMV per row. Q4_0 and Q8_0 need m (rounded up to 64)
  * * cols * 2 < 2^31 (their kernels address the f16 activation rows by 32-bit
  * byte offsets); larger calls return hipErrorInvalidValue.
  * Scratch: the matrix-core calls and the decode attentions that allocate keep what they

@@ -37,6 +37,28 @@ __device__ inline f4_t mfma32(h8_t a, h8_t b, f4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
+// The 16x16x4 f32 MFMA: lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16]; D as above.
+__device__ inline f4_t mfma4(float a, float b, f4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// The sum of n K-split partials: pairs, pairs of pairs, then the groups of four in order.
+// One after another, 16 or 32 roundings at the sum's own size were a third of a product's
+// error (9 rows, 1024 x 14336 Q8_0, 32 splits: 1.41e-7 of the result).
+template <class V, class F>
+__device__ inline V split_sum(int n, F&& load) {
+  V s = {};
+  for (int z = 0; z < n; z += 4) {
+    const int m = n - z;  // at least 1
+    V a = load(z), b = {}, c = {}, d = {};
+    if (m > 1) b = load(z + 1);
+    if (m > 2) c = load(z + 2);
+    if (m > 3) d = load(z + 3);
+    s += (a + b) + (c + d);
+  }
+  return s;
+}
+
 __device__ inline float pow2f_i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 
 // 16 bytes per lane from a wave-uniform base (scalar registers) plus the lane's

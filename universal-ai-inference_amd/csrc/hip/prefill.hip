@@ -40,8 +40,15 @@ __global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t l
   uint2* lo2 = reinterpret_cast<uint2*>(act.lo);
   // float4 i of the row: quad i % 8 of 32-block i / 8, in the order 0, 4, 1, 5, ...
   auto at = [&](int i) -> int64_t { return ((int64_t)(i >> 3) * act.mpad + t) * 8 + 2 * (i & 3) + ((i >> 2) & 1); };
+  float4* raw4 = reinterpret_cast<float4*>(act.raw);
+  auto raw_at = [&](int i) -> int64_t {
+    return (((int64_t)((i >> 2) & 1) * (K / 32) + (i >> 3)) * act.mpad + t) * 4 + (i & 3);
+  };
   if (t >= M) {
-    for (int i = tid; i < nv; i += NT) { hi2[at(i)] = make_uint2(0, 0); lo2[at(i)] = make_uint2(0, 0); }
+    for (int i = tid; i < nv; i += NT) {
+      if (act.hi) hi2[at(i)] = lo2[at(i)] = make_uint2(0, 0);
+      if (act.raw) raw4[raw_at(i)] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
     if (act.sxp) {
       for (int i = tid; i < nv / 8; i += NT)
         reinterpret_cast<uint2*>(act.sxp)[((int64_t)(i >> 3) * act.mpad + t) * 8 + (i & 7)] = make_uint2(0, 0);
@@ -55,12 +62,10 @@ __global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t l
   for (int i = tid; i < nv; i += NT) {
     float4 v = x4[i];
     if (nsplit > 0) {
-      // residual add of a K-split GEMM's partials, in split order
-      float4 p = reinterpret_cast<const float4*>(part + t * ldx)[i];
-      for (int z = 1; z < nsplit; ++z) {
-        const float4 q = reinterpret_cast<const float4*>(part + ((int64_t)z * M + t) * ldx)[i];
-        p.x += q.x; p.y += q.y; p.z += q.z; p.w += q.w;
-      }
+      // residual add of a K-split GEMM's partials
+      const f4_t p = split_sum<f4_t>(nsplit, [&](int z) {
+        return reinterpret_cast<const f4_t*>(part + ((int64_t)z * M + t) * ldx)[i];
+      });
       v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
       x4[i] = v;
     }
@@ -90,6 +95,10 @@ __global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t l
       amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
     }
     __syncthreads();  // red[] is reused below
+  }
+  if (act.raw) {
+    for (int i = tid; i < nv; i += NT) raw4[raw_at(i)] = r4[i];
+    if (!act.hi) return;
   }
   amax = wave_max(amax);
   if ((tid & 63) == 0) red[tid >> 6] = amax;
@@ -149,12 +158,9 @@ __global__ void __launch_bounds__(256) k_pf_qkv(PfQkvArgs a) {
   const int pos = a.p0 + (int)t;
   const float* row = a.qkv + t * a.ldq;
   // value x of this row: the GEMM's output, or the sum of its K-split partials
-  // in split order
   auto val = [&](int x) -> float {
     if (a.nsplit <= 1) return row[x];
-    float v = a.part[t * a.ldq + x];
-    for (int z = 1; z < a.nsplit; ++z) v = v + a.part[((int64_t)z * a.M + t) * a.ldq + x];
-    return v;
+    return split_sum<float>(a.nsplit, [&](int z) { return a.part[((int64_t)z * a.M + t) * a.ldq + x]; });
   };
   const int hd = a.head_dim, half = hd / 2;
   const int npair = (a.q_dim + a.kv_dim) / 2;

@@ -2,10 +2,21 @@
 // cores (quant_gemm_f32, libs/uaii-quant/src/quant_gemm.cpp:22-70: per weight row,
 // dequantise to f32 and dot with every activation row).
 //
-// The activations come from k_pf_prep as f16 pairs hi + lo (about 22 significant
-// bits), the weights as small integers that f16 holds exactly, decoded in
-// registers from their split GGUF layout; v_mfma_f32_16x16x32_f16 multiplies the
-// integers with hi and with lo and sums in f32.
+// For the quantised formats the activations come from k_pf_prep as f16 pairs hi + lo
+// (about 22 significant bits), the weights as small integers that f16 holds exactly,
+// decoded in registers from their split GGUF layout; v_mfma_f32_16x16x32_f16 multiplies
+// the integers with hi and with lo and sums in f32.
+//
+// F16 weights take the f32 rows and v_mfma_f32_16x16x4_f32 (157 TFLOP/s dense, a
+// sixteenth of the f16 rate). As f16 pairs their products, whose exponents spread, lost
+// more to the f16 op's sums than one GEMV per row does (1.05e-7 of the result against
+// 0.83e-7 at K = 512; 1.5e-6 against 0.85e-7 with subnormal weights), and infinities met
+// zeros. Now eight products make a sum, four sums are added in pairs, and the running sum
+// carries what it lost to rounding beside it: 0.72e-7 at every K up to 14336 and
+// 0.77e-7 .. 0.99e-7 with K splits, where the GEMV has 0.83e-7 .. 1.07e-7. 1024 rows of
+// 4096 x 4096 104 -> 359 us, 9 rows 16.4 -> 19.5 (one row at a time 7.0 ms and 64 us); the
+// matrix ops and the sums' vector work beside them bound it (95 TFLOP/s; 112 with one
+// sum a block and plain additions, whose error was 1.0e-7).
 //
 // What bounds it. With many rows, vector and LDS work beside the matrix ops: a probe
 // of f16 matrix ops (two waves per SIMD, nothing loaded from memory) sustained 1.9
@@ -15,8 +26,8 @@
 // column subtiles of the wave, so NT = 4 halves the reads of the 64 x 32 wave tile
 // used before; the integers' hi and lo products count twice, so 1.1 PFLOP/s of matrix
 // ops are 0.55 of the product's. Measured on 1024 rows, 28672 x 4096 (TFLOP/s, before
-// and now): Q4_0 453, 481; Q8_0 386, 430; Q4_K 266, 455; Q6_K 186, 347; on Q5_K 400
-// and F16 368, which ran one row at a time. With few rows the launch is a chain of
+// and now): Q4_0 453, 481; Q8_0 386, 430; Q4_K 266, 455; Q6_K 186, 347; on Q5_K 400,
+// which ran one row at a time. With few rows the launch is a chain of
 // round trips to memory; a K split and smaller blocks shorten it: 9 rows, 4096 x 4096,
 // with the preparation and the fold (us): Q4_0 47, 17; Q8_0 52, 19; Q4_K 88, 17;
 // Q6_K 120, 20.
@@ -130,8 +141,13 @@ __device__ inline void decode_block(const Words<FMT>& r, const Unit<FMT>& u, int
     b = cat8(as_h2(byte_pair(v0)) + c, as_h2(byte_pair(v0 >> 8)) + c, as_h2(byte_pair(v1)) + c,
              as_h2(byte_pair(v1 >> 8)) + c);
   } else if constexpr (FMT == T_F16) {
-    b = cat8(as_h2(__builtin_amdgcn_perm(r.w[1], r.w[0], 0x05040100u)), as_h2(__builtin_amdgcn_perm(r.w[1], r.w[0], 0x07060302u)),
-             as_h2(__builtin_amdgcn_perm(r.w[3], r.w[2], 0x05040100u)), as_h2(__builtin_amdgcn_perm(r.w[3], r.w[2], 0x07060302u)));
+    // the f32 values of quad g (b) and quad 4 + g (blo)
+    auto quad = [&](uint32_t u, uint32_t v) __attribute__((always_inline)) {
+      const h2_t p = as_h2(u), q = as_h2(v);
+      return __builtin_bit_cast(h8_t, f4_t{(float)p.x, (float)p.y, (float)q.x, (float)q.y});
+    };
+    b = quad(r.w[0], r.w[1]);
+    blo = quad(r.w[2], r.w[3]);
   } else if constexpr (FMT == T_Q4_K || FMT == T_Q5_K) {
     const int j = 2 * h + t;  // sub-block: the stage's low (t = 0) or high nibbles
     const uint32_t w0 = r.w[0], w1 = r.w[1];
@@ -236,8 +252,9 @@ __device__ inline __attribute__((always_inline)) void for_n(F&& f) {
 template <int FMT, int EPI, int MT, int KH>
 __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
   constexpr int NT = nt_of<FMT>();
-  constexpr bool BLOCK_SCALE = !is_k<FMT>();  // f32 sums per 32-block (F16: for their accuracy)
-  constexpr bool TWO = FMT != T_Q4_0;         // sums per 256 k, then over K
+  constexpr bool F32 = FMT == T_F16;          // f32 operands
+  constexpr bool BLOCK_SCALE = !is_k<FMT>() && !F32;  // f32 sums per 32-block
+  constexpr bool TWO = FMT != T_Q4_0 && !F32;  // sums per 256 k, then over K
   using L = Lds<FMT, MT>;
   constexpr int BM = 16 * MT;
   constexpr int NQ = (EPI == EPI_SWIGLU) ? NT / 2 : NT;  // distinct row subtiles
@@ -394,7 +411,7 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
   };
 
   const f4_t zero = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  f4_t acc[MT][NT], part[MT][NT];
+  f4_t acc[MT][NT], part[MT][NT];  // F32: part is what acc lost to rounding
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -584,6 +601,27 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
           }
         }
         psc = sc;
+      } else if constexpr (F32) {
+        // four sums of 8 values (two matrix ops each), added in pairs
+        const f4_t bq[2] = {__builtin_bit_cast(f4_t, bc), __builtin_bit_cast(f4_t, bcl)};
+        f4_t s8[4][MT];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+#pragma unroll
+          for (int i = 0; i < MT; ++i)
+            s8[e >> 1][i] = mfma4(__builtin_bit_cast(f4_t, fa[i][e >> 2])[e & 3], bq[e >> 2][e & 3],
+                                  (e & 1) == 0 ? zero : s8[e >> 1][i]);
+          if (e == 3) next_frags(0);
+        }
+        next_frags(1);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const f4_t add = (s8[0][i] + s8[1][i]) + (s8[2][i] + s8[3][i]), to = acc[i][j] + add;
+          part[i][j] += add - (to - acc[i][j]);
+          acc[i][j] = to;
+          pin(acc[i][j]);
+          pin(part[i][j]);
+        }
       } else {
         constexpr bool first = h == 0 && t == 0;  // of the unit
 #pragma unroll
@@ -640,6 +678,16 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
     }
   }
 
+  if constexpr (F32) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)  // an infinite sum has nothing beside it
+          if (isfinite(acc[i][j][r])) acc[i][j][r] += part[i][j][r];
+  }
+
   if constexpr (KH == 2) {
     __builtin_amdgcn_s_waitcnt(0x0070);
     __syncthreads();
@@ -666,7 +714,7 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
     for (int r = 0; r < 4; ++r) {
       const int64_t t = mr.m0 + 16 * i + 4 * g + r;
       if (t >= mr.mend) continue;
-      const float rs = a.rs[arow(t)];
+      const float rs = F32 ? 1.0f : a.rs[arow(t)];
       float* yrow = a.y + t * a.ldy + seg.col0;
       float* prw = split ? a.part + ((int64_t)blockIdx.z * a.M + t) * a.ldp + seg.col0 : nullptr;
 #pragma unroll
@@ -693,7 +741,7 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
   }
 }
 
-// The partials of a K-split launch, added in split order, and the epilogue:
+// The partials of a K-split launch, added up (split_sum), and the epilogue:
 // y [M][ldy] from part [ksplit][M][ldp]; SwiGLU's gate and up sums side by side.
 // Block: 256 V-wide pieces of row blockIdx.y.
 template <int EPI, int V>
@@ -704,13 +752,9 @@ __global__ void __launch_bounds__(256) k_pf_fold(const float* __restrict__ part,
   if (n >= N) return;
   const float* p = part + t * ldp + n;
   const int64_t zs = M * ldp;
-  vec v = *reinterpret_cast<const vec*>(p), u;
-  if constexpr (EPI == EPI_SWIGLU) u = *reinterpret_cast<const vec*>(p + N);
-#pragma unroll 8  // the loads of eight partials in flight at once
-  for (int z = 1; z < ksplit; ++z) {
-    v += *reinterpret_cast<const vec*>(p + z * zs);
-    if constexpr (EPI == EPI_SWIGLU) u += *reinterpret_cast<const vec*>(p + z * zs + N);
-  }
+  const auto at = [&](int64_t o) { return *reinterpret_cast<const vec*>(p + o); };
+  vec v = split_sum<vec>(ksplit, [&](int z) { return at(z * zs); }), u;
+  if constexpr (EPI == EPI_SWIGLU) u = split_sum<vec>(ksplit, [&](int z) { return at(z * zs + N); });
   vec* o = reinterpret_cast<vec*>(y + t * ldy + n);
   if constexpr (EPI == EPI_ADD) v += *o;
 #pragma unroll

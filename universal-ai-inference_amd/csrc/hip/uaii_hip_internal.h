@@ -254,10 +254,14 @@ hipError_t launch_argmax_final(float* part_val, int32_t* part_idx, int nparts, S
 // decode (prefill_gemm.hip). sxp: per 256 k a block of the same shape holding the
 // sums of x * 2^(e - 5) over the eight 32-blocks as f16 parts (eight first parts,
 // eight second, eight third, eight zeros; together all 24 bits).
+// raw: the rows as they are, for F16 weights, whose products are f32: a block's values
+// 0..15 of all rows ([K / 32][mpad][16]), then the same of the values 16..31.
+// What no consumer takes is null.
 struct PfAct {
   __half* hi;
   __half* lo;
-  __half* sxp;    // [K / 256][mpad][32], or null where no consumer takes it
+  __half* sxp;    // [K / 256][mpad][32]
+  float* raw;     // [2][K / 32][mpad][16]
   float* rs;      // [mpad]
   int64_t mpad;   // rows allocated (pf_mpad); rows >= M are zero
   int64_t K;
@@ -276,7 +280,7 @@ struct PfGemmArgs {
   int nseg;
   int epi;              // EPI_STORE, EPI_ADD, EPI_SWIGLU, EPI_GELU
   int64_t M, K, mpad;
-  const __half* ahi;
+  const __half* ahi;    // F16 weights: the two halves of PfAct::raw
   const __half* alo;
   const __half* sxp;    // Q4_K, Q5_K
   const float* rs;
@@ -284,7 +288,7 @@ struct PfGemmArgs {
   int64_t ldy;
   // ksplit > 1: blocks along grid z each take a share of K and store their sums to
   // part[z][M][ldp] (EPI_SWIGLU: gate and up sums side by side) instead of the
-  // epilogue, which launch_pf_fold or the next kernel to read y does, z in order
+  // epilogue, which launch_pf_fold or the next kernel to read y does (split_sum)
   int ksplit;
   float* part;
   int64_t ldp;
@@ -348,6 +352,18 @@ bool pf_router_supported(int type);
 
 bool pf_supported(int type);
 bool pf_k_quant(int type);  // rows are whole 256-value super-blocks
+// What the row GEMM of a weight format reads of its activations.
+enum : int { PF_SPLIT = 1, PF_SUMS = 2, PF_RAW = 4 };  // hi + lo; sxp; raw
+inline int pf_reads(int type) {
+  return type == T_F16 ? PF_RAW : type == T_Q4_K || type == T_Q5_K ? PF_SPLIT | PF_SUMS : PF_SPLIT;
+}
+// The two activation pointers of a row GEMM of that format.
+inline void pf_take(const PfAct& act, int type, PfGemmArgs* a) {
+  a->ahi = type == T_F16 ? reinterpret_cast<const __half*>(act.raw) : act.hi;
+  a->alo = type == T_F16 ? reinterpret_cast<const __half*>(act.raw + act.mpad * a->K / 2) : act.lo;
+  a->sxp = act.sxp;
+  a->rs = act.rs;
+}
 // The formats that prefill() takes and whose row GEMM reports what it cannot run; the
 // others' callers ran token by token or row by row before, and fall back to that.
 bool pf_required(int type);

@@ -217,18 +217,17 @@ int gemm_common(const uaii_hip_weight* w, const uaii_hip_weight* w2, const float
   if (e != hipSuccess) return (int)e;
   char* base = scratch->data();
   PfAct act{};
-  act.hi = reinterpret_cast<__half*>(base);
-  act.lo = reinterpret_cast<__half*>(base + hb);
-  act.sxp = (v.type == T_Q4_K || v.type == T_Q5_K) ? reinterpret_cast<__half*>(base + 2 * hb) : nullptr;
+  const int reads = pf_reads(v.type);
+  if (reads & PF_RAW) act.raw = reinterpret_cast<float*>(base);
+  if (reads & PF_SPLIT) act.hi = reinterpret_cast<__half*>(base);
+  if (reads & PF_SPLIT) act.lo = reinterpret_cast<__half*>(base + hb);
+  if (reads & PF_SUMS) act.sxp = reinterpret_cast<__half*>(base + 2 * hb);
   act.rs = reinterpret_cast<float*>(base + 2 * hb + xb);
   act.mpad = mpad;
   act.K = K;
   e = launch_pf_prep(const_cast<float*>(x), K, m, norm_w, eps, act, S(stream));
   if (e != hipSuccess) return (int)e;
-  a.ahi = act.hi;
-  a.alo = act.lo;
-  a.sxp = act.sxp;
-  a.rs = act.rs;
+  pf_take(act, v.type, &a);
   a.part = reinterpret_cast<float*>(base + 2 * hb + xb + rb);
   e = launch_pf_gemm(a, S(stream));
   if (e != hipSuccess || a.ksplit <= 1) return (int)e;

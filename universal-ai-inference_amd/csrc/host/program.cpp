@@ -364,6 +364,7 @@ Error DecoderProgram::build(const DecoderSpec& spec, const ProgramOptions& opts)
     for (const DeviceWeight* w : ws) {
       rows = rows && pf_supported(w->view.type);
       required = required && pf_required(w->view.type);
+      pf_reads_ |= pf_reads(w->view.type);
     }
   }
   if (const char* env = std::getenv("UAII_PREFILL")) {
@@ -453,9 +454,12 @@ Error DecoderProgram::ensure_prefill_buffers(int64_t chunk) {
     UAII_TRY(alloc(4 * CK * (size_t)inter, (void**)&pf_h_));
     if (inter_sh > 0) UAII_TRY(alloc(4 * C * (size_t)inter_sh, (void**)&pf_hsh_));
   }
-  UAII_TRY(alloc(2 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.hi));
-  UAII_TRY(alloc(2 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.lo));
-  UAII_TRY(alloc(64 * (size_t)((kmax + 255) / 256) * (size_t)mpad, (void**)&pf_act_.sxp));
+  if (pf_reads_ & PF_SPLIT) {
+    UAII_TRY(alloc(2 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.hi));
+    UAII_TRY(alloc(2 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.lo));
+  }
+  if (pf_reads_ & PF_SUMS) UAII_TRY(alloc(64 * (size_t)((kmax + 255) / 256) * (size_t)mpad, (void**)&pf_act_.sxp));
+  if (pf_reads_ & PF_RAW) UAII_TRY(alloc(4 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.raw));
   UAII_TRY(alloc(4 * (size_t)mpad, (void**)&pf_act_.rs));
   pf_act_.mpad = mpad;
   pf_act_rows_ = mpad;
@@ -475,10 +479,7 @@ Error DecoderProgram::pf_gemm(const DeviceWeight* w[3], const int64_t cols0[3], 
     a.M = m;
     a.K = w[i]->view.cols;
     a.mpad = pf_act_.mpad;
-    a.ahi = pf_act_.hi;
-    a.alo = pf_act_.lo;
-    a.sxp = pf_act_.sxp;
-    a.rs = pf_act_.rs;
+    pf_take(pf_act_, w[i]->view.type, &a);
     a.y = y;
     a.ldy = ldy;
     int j = i;
@@ -545,13 +546,15 @@ int DecoderProgram::pf_store_split(const DeviceWeight* w[3], int nw, int64_t m, 
   return (int)std::max<int64_t>(1, std::min<int64_t>(ks, pf_part_floats_ / std::max<int64_t>(m * ldy, 1)));
 }
 
-Error DecoderProgram::pf_prep(float* x, int64_t K, int64_t m, const float* norm_w, bool sums) {
+Error DecoderProgram::pf_prep(float* x, int64_t K, int64_t m, const float* norm_w, int reads) {
   if (pf_mpad(m) > pf_act_rows_ || K > pf_kmax_)
     return Error::make(ErrorCode::Internal, "prefill activation rows exceed their buffer");
   pf_act_.mpad = pf_mpad(m);
   PfAct act = pf_act_;
   act.K = K;
-  if (!sums) act.sxp = nullptr;
+  if (!(reads & PF_SPLIT)) act.hi = act.lo = nullptr;
+  if (!(reads & PF_SUMS)) act.sxp = nullptr;
+  if (!(reads & PF_RAW)) act.raw = nullptr;
   const int pend = (x == pf_x_) ? pf_pending_ : 0;
   UAII_HIP(launch_pf_prep(x, K, m, norm_w, spec_.rms_eps, act, stream_, pend ? pf_part_ : nullptr, pend));
   if (pend) pf_pending_ = 0;
@@ -570,8 +573,8 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
   const int E = (int)d.n_experts;
   const int k = (int)std::min<int64_t>(d.top_k, d.n_experts);
   const int64_t I = ls.inter;
-  auto sums = [](const DeviceWeight& w) { return w.view.type == T_Q4_K || w.view.type == T_Q5_K; };
-  UAII_TRY(prep(pf_x_, d.dim, m, L.ffn_norm, sums(L.gate_exps) || (L.shared && sums(L.gate_sh))));
+  auto reads = [](const DeviceWeight& w) { return pf_reads(w.view.type); };
+  UAII_TRY(prep(pf_x_, d.dim, m, L.ffn_norm, reads(L.gate_exps) | (L.shared ? reads(L.gate_sh) : 0)));
   UAII_TRY(timed("pf_moe_route", 4.0 * (double)(m * d.dim + E * d.dim), 2.0 * (double)(m * E * d.dim), [&] {
     return launch_pf_moe_route(pf_x_, m, d.dim, L.ffn_norm, d.rms_eps, L.gate_inp.view, E, k, pf_moe_ids_,
                                pf_moe_w_, s);
@@ -609,17 +612,15 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
   if ((int64_t)tab.size() > pf_tab_cap_)
     return Error::make(ErrorCode::Internal, "MoE prefill row table exceeds its buffer");
   UAII_HIP(hipMemcpyAsync(pf_moe_tab_, tab.data(), 4 * tab.size(), hipMemcpyHostToDevice, s));
-  auto grouped = [&](int64_t K, int epi, int bm, int t0, int nt) {
+  auto grouped = [&](const DeviceWeight& w, int64_t K, int epi, int bm, int t0, int nt) {
     PfGemmArgs g{};
     g.nseg = 1;
     g.epi = epi;
     g.M = m * k;
     g.K = K;
     g.mpad = pf_mpad(m * k);
-    g.ahi = pf_act_.hi;
-    g.alo = pf_act_.lo;
-    g.sxp = pf_act_.sxp;
-    g.rs = pf_act_.rs;
+    g.seg[0].w = w.view;
+    pf_take(pf_act_, w.view.type, &g);
     g.act_ld = pf_act_.mpad;
     g.gtab = pf_moe_tab_ + 3 * t0;
     g.ntab = nt;
@@ -629,11 +630,10 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
   };
   {
     // gathered token rows x gate / up of their experts -> routed hidden rows
-    PfGemmArgs g = grouped(d.dim, EPI_SWIGLU, bm_gu, t_gu, n_gu);
+    PfGemmArgs g = grouped(L.gate_exps, d.dim, EPI_SWIGLU, bm_gu, t_gu, n_gu);
     g.arow = pf_moe_list_;
     g.y = pf_h_;
     g.ldy = I;
-    g.seg[0].w = L.gate_exps.view;
     g.seg[0].w2 = L.up_exps.view;
     g.seg[0].rows = I;
     const double bytes = 2.0 * (double)L.gate_exps.bytes * n_used / E;
@@ -645,12 +645,11 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
     UAII_TRY(gemm("pf_gemm_shared_gate_up", wg, c00, 1, &L.up_sh, EPI_SWIGLU, m, pf_hsh_, L.inter_sh));
   }
   // the routed tokens' hidden rows, packed by expert
-  UAII_TRY(prep(pf_h_, I, m * k, nullptr, sums(L.down_exps)));
+  UAII_TRY(prep(pf_h_, I, m * k, nullptr, reads(L.down_exps)));
   {
-    PfGemmArgs g = grouped(I, EPI_STORE, bm_dn, t_dn, n_dn);
+    PfGemmArgs g = grouped(L.down_exps, I, EPI_STORE, bm_dn, t_dn, n_dn);
     g.y = pf_moe_y_;
     g.ldy = d.dim;
-    g.seg[0].w = L.down_exps.view;
     g.seg[0].rows = d.dim;
     const double bytes = (double)L.down_exps.bytes * n_used / E;
     UAII_TRY(timed("pf_moe_down", bytes, 2.0 * (double)(m * k * I * d.dim), [&] { return launch_pf_gemm(g, s); }));
@@ -659,7 +658,7 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
     return launch_pf_moe_combine(pf_x_, m, d.dim, k, pf_moe_w_, pf_moe_inv_, pf_moe_y_, s);
   }));
   if (L.shared) {
-    UAII_TRY(prep(pf_hsh_, L.inter_sh, m, nullptr, sums(L.down_sh)));
+    UAII_TRY(prep(pf_hsh_, L.inter_sh, m, nullptr, reads(L.down_sh)));
     const DeviceWeight* wd[3] = {&L.down_sh, nullptr, nullptr};
     UAII_TRY(gemm("pf_gemm_shared_down", wd, c00, 1, nullptr, EPI_ADD, m, pf_x_, d.dim));
   }
@@ -721,10 +720,10 @@ Error DecoderProgram::prefill_rows(int64_t n) {
   const size_t layer_kv = (size_t)d.kv_dim * (size_t)max_ctx_ * (opts_.kv_f16 ? 2 : 4);
   const int64_t ldqkv = d.q_dim + 2 * d.kv_dim;
   prof_used_ = 0;
-  auto prep = [&](float* x, int64_t K, int64_t m, const float* norm_w, bool sums) -> Error {
+  auto prep = [&](float* x, int64_t K, int64_t m, const float* norm_w, int reads) -> Error {
     Error err = Error::success();
     Error launched = timed("pf_prep", 12.0 * (double)m * (double)K, 0.0, [&]() -> hipError_t {
-      err = pf_prep(x, K, m, norm_w, sums);
+      err = pf_prep(x, K, m, norm_w, reads);
       return err.ok() ? hipSuccess : hipErrorInvalidValue;
     });
     if (!err.ok()) return err;
@@ -769,10 +768,10 @@ Error DecoderProgram::prefill_rows(int64_t n) {
       const LayerSpec& ls = d.layers[(size_t)li];
       uint8_t* kbase = static_cast<uint8_t*>(kv_) + (size_t)li * 2 * layer_kv;
       uint8_t* vbase = kbase + layer_kv;
-      // a prep's per-32 sums, where a GEMM reading it takes them
-      auto sums = [](const DeviceWeight& w) { return w.view.type == T_Q4_K || w.view.type == T_Q5_K; };
+      // what the GEMMs that follow a prep read of it
+      auto reads = [](const DeviceWeight& w) { return pf_reads(w.view.type); };
       // attention block (gguf.cpp:1000-1060)
-      UAII_TRY(prep(pf_x_, d.dim, m, L.attn_norm, sums(L.wq) || sums(L.wk) || sums(L.wv)));
+      UAII_TRY(prep(pf_x_, d.dim, m, L.attn_norm, reads(L.wq) | reads(L.wk) | reads(L.wv)));
       const DeviceWeight* qkv[3] = {&L.wq, &L.wk, &L.wv};
       const int64_t qkv_cols[3] = {0, d.q_dim, d.q_dim + d.kv_dim};
       const int qkv_split = pf_store_split(qkv, 3, m, ldqkv);
@@ -817,13 +816,13 @@ Error DecoderProgram::prefill_rows(int64_t n) {
       UAII_TRY(timed("pf_attention", 4.0 * pairs * (double)d.kv_dim, 4.0 * pairs * (double)d.q_dim, [&] {
         return opts_.kv_f16 ? launch_pf_attn(at, s) : launch_pf_attn_f32(at, s);
       }));
-      UAII_TRY(prep(pf_attn_, d.q_dim, m, nullptr, sums(L.wo)));
+      UAII_TRY(prep(pf_attn_, d.q_dim, m, nullptr, reads(L.wo)));
       const DeviceWeight* wo[3] = {&L.wo, nullptr, nullptr};
       const int64_t c00[3] = {0, 0, 0};
       UAII_TRY(gemm("pf_gemm_o", wo, c00, 1, nullptr, EPI_ADD, m, pf_x_, d.dim));
       // FFN block (gguf.cpp:1130-1173)
       if (ls.ffn == LayerSpec::kSwiGLU || ls.ffn == LayerSpec::kGelu) {
-        UAII_TRY(prep(pf_x_, d.dim, m, L.ffn_norm, sums(L.up)));  // gate and up share a format
+        UAII_TRY(prep(pf_x_, d.dim, m, L.ffn_norm, reads(L.up)));  // gate and up share a format
         if (ls.ffn == LayerSpec::kSwiGLU) {
           const DeviceWeight* wg[3] = {&L.gate, nullptr, nullptr};
           UAII_TRY(gemm("pf_gemm_gate_up", wg, c00, 1, &L.up, EPI_SWIGLU, m, pf_h_, ls.inter));
@@ -831,7 +830,7 @@ Error DecoderProgram::prefill_rows(int64_t n) {
           const DeviceWeight* wu[3] = {&L.up, nullptr, nullptr};
           UAII_TRY(gemm("pf_gemm_up", wu, c00, 1, nullptr, EPI_GELU, m, pf_h_, ls.inter));
         }
-        UAII_TRY(prep(pf_h_, ls.inter, m, nullptr, sums(L.down)));
+        UAII_TRY(prep(pf_h_, ls.inter, m, nullptr, reads(L.down)));
         const DeviceWeight* wd[3] = {&L.down, nullptr, nullptr};
         UAII_TRY(gemm("pf_gemm_down", wd, c00, 1, nullptr, EPI_ADD, m, pf_x_, d.dim));
       } else if (ls.ffn == LayerSpec::kMoE) {

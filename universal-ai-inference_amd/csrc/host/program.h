@@ -153,7 +153,7 @@ class DecoderProgram {
   Error pf_gemm(const DeviceWeight* w[3], const int64_t cols0[3], int nw, const DeviceWeight* w2,
                 int epi, int64_t m, float* y, int64_t ldy, int store_split = 1);
   int pf_store_split(const DeviceWeight* w[3], int nw, int64_t m, int64_t ldy);
-  Error pf_prep(float* x, int64_t K, int64_t m, const float* norm_w, bool sums);
+  Error pf_prep(float* x, int64_t K, int64_t m, const float* norm_w, int reads);
   template <class Prep, class Gemm>
   Error prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m, Prep&& prep, Gemm&& gemm);
   Error encode_step(bool want_logits);
@@ -217,6 +217,7 @@ class DecoderProgram {
   // prefill: chunk buffers ([chunk][...] rows) and the prepared-activation scratch
   bool pf_ok_ = false;    // prefill(): the weights' formats (pf_required) and an f16 cache
   bool pf_rows_ = false;  // generate_rows(): the weights' formats
+  int pf_reads_ = 0;      // what their row GEMMs read of the activations (pf_reads)
   int64_t pf_chunk_ = 0, pf_kmax_ = 0;
   float *pf_x_ = nullptr, *pf_qkv_ = nullptr, *pf_q_ = nullptr, *pf_attn_ = nullptr,
         *pf_h_ = nullptr;
