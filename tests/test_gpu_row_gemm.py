@@ -164,3 +164,32 @@ def test_f16_rows_infinities(hip):
         ok = np.isfinite(want[i])
         if ok.any():
             assert np.abs(got[i][ok] - want[i][ok]).max() <= 4e-6 * np.abs(want[i][ok]).max(), i
+
+
+@pytest.mark.parametrize("t", [t for t in TYPES if t != uaii_amd.F16], ids=lambda t: uaii_amd.TYPE_NAMES[t])
+def test_row_gemm_extreme_rows(hip, t):
+    """Rows of finite values near the largest and the smallest f32 holds, beside an
+    ordinary one: each keeps its precision (the row's power-of-two scale)."""
+    m, rows, cols = 5, 70, 512
+    w, wf = weights(t, rows, cols, 21)
+    x = synth.normals(21, 2, 0, m * cols, 1.0).reshape(m, cols)
+    # |x| up to about 4 of each: past 2^115 and near 2^127; below 2^-100 and near 2^-126
+    x *= np.float32([1, 2e35, 4e37, 1e-31, 1e-36])[:, None]
+    dx, dy = DeviceBuffer.from_array(x), DeviceBuffer(4 * m * rows)
+    check_hip(hip.uaii_hip_gemm(w.h, dx.ptr, m, dy.ptr, None))
+    check_hip(hip.uaii_hip_synchronize())
+    got, want = dy.to_array(np.float32, m * rows).reshape(m, rows), x.astype(np.float64) @ wf.T
+    err = np.abs(got - want).max(1) / np.abs(want).max(1)
+    print(uaii_amd.TYPE_NAMES[t], err, flush=True)
+    assert (err < 4e-6).all()
+
+
+def test_row_gemm_infinite_activation(hip):
+    """An infinite activation of a Q8_0 product gives what it gives one row at a time."""
+    m, rows, cols = 4, 70, 512
+    w, wf = weights(uaii_amd.Q8_0, rows, cols, 22)
+    x = synth.normals(22, 2, 0, m * cols, 1.0).reshape(m, cols)
+    x[1, 100], x[2, 3] = np.inf, -np.inf
+    got, want = rows_and_steps(hip, w, x, rows)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    assert np.array_equal(got[np.isinf(got)], want[np.isinf(want)]) and np.isinf(got[1]).sum() > rows // 2

@@ -106,11 +106,12 @@ __global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t l
 #pragma unroll
   for (int w = 0; w < NT / 64; ++w) amax = fmaxf(amax, red[w]);
   // scale so that max |x| * 2^e lies in [2^14, 2^15): hi keeps 11 bits of every
-  // element near the top of the row and lo the next 11
+  // element near the top of the row and lo the next 11. The limits are where 2^e and
+  // 2^-e are normal numbers and the largest finite row still fits f16.
   int e = 0;
   if (amax > 0.0f) {
     const int ex = (int)((__float_as_uint(amax) >> 23) & 0xff) - 126;  // amax in [2^(ex-1), 2^ex)
-    e = min(100, max(-100, 15 - ex));
+    e = min(126, max(-113, 15 - ex));
   }
   const float s = pow2f_i(e);
   if (tid == 0) act.rs[t] = pow2f_i(-e);
@@ -121,8 +122,9 @@ __global__ void __launch_bounds__(NT) k_pf_prep(float* __restrict__ x, int64_t l
       const float4 v = r4[i];
       const float y0 = v.x * s, y1 = v.y * s, y2 = v.z * s, y3 = v.w * s;
       const _Float16 h0 = (_Float16)y0, h1 = (_Float16)y1, h2 = (_Float16)y2, h3 = (_Float16)y3;
-      const _Float16 l0 = (_Float16)(y0 - (float)h0), l1 = (_Float16)(y1 - (float)h1);
-      const _Float16 l2 = (_Float16)(y2 - (float)h2), l3 = (_Float16)(y3 - (float)h3);
+      // an infinity is all in hi
+      auto rest = [](float y, _Float16 h) { return (_Float16)(fabsf(y) == INFINITY ? 0.0f : y - (float)h); };
+      const _Float16 l0 = rest(y0, h0), l1 = rest(y1, h1), l2 = rest(y2, h2), l3 = rest(y3, h3);
       // stored order (k0, k2, k1, k3)
       hi2[at(i)] = make_uint2(__builtin_bit_cast(uint32_t, h2_t{h0, h2}),
                           __builtin_bit_cast(uint32_t, h2_t{h1, h3}));
