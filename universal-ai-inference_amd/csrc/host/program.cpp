@@ -134,6 +134,18 @@ Error DecoderProgram::charge(uint64_t& pool, uint64_t bytes) {
   return Error::success();
 }
 
+// Device memory that the session cannot do without: the same buffers give way where the
+// device has no room beside them.
+hipError_t DecoderProgram::device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory || pf_ok_ || used_pf_ == 0) return e;
+  (void)hipGetLastError();
+  e = hipStreamSynchronize(stream_);
+  if (e != hipSuccess) return e;
+  release_prefill_buffers();
+  return hipMalloc(p, bytes);
+}
+
 // The load of a weight whose bytes the file does not hold fails as the
 // reference's load_or_init_weights does (session.cpp:510-544): an error unless
 // weight_init asks for a synthetic fill of the f32 buffer (zeros, ones, or
@@ -865,14 +877,14 @@ Error DecoderProgram::ensure_capacity(int64_t max_seq) {
   const size_t part = (size_t)d.n_kv_heads * attn_splits_ * G * (size_t)(hd + 2);
   UAII_TRY(charge(used_dyn_, kv_bytes_ + kv_slack + sizeof(int32_t) * (size_t)(max_seq + 2) +
                                  sizeof(float2) * (size_t)max_seq * (size_t)(hd / 2) + part * 4));
-  UAII_HIP(hipMalloc(&kv_, kv_bytes_ + kv_slack));
+  UAII_HIP(device_malloc((void**)&kv_, kv_bytes_ + kv_slack));
   UAII_HIP(hipMemsetAsync(kv_, 0, kv_bytes_ + kv_slack, stream_));
-  UAII_HIP(hipMalloc((void**)&ids_, sizeof(int32_t) * (size_t)(max_seq + 2)));
+  UAII_HIP(device_malloc((void**)&ids_, sizeof(int32_t) * (size_t)(max_seq + 2)));
   UAII_HIP(hipMemsetAsync(ids_, 0, sizeof(int32_t) * (size_t)(max_seq + 2), stream_));
   std::vector<float2> tab = rope_table(d.rope_theta, hd, max_seq);
-  UAII_HIP(hipMalloc((void**)&rope_, tab.size() * sizeof(float2)));
+  UAII_HIP(device_malloc((void**)&rope_, tab.size() * sizeof(float2)));
   UAII_HIP(hipMemcpy(rope_, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice));
-  UAII_HIP(hipMalloc((void**)&attn_part_, part * 4));
+  UAII_HIP(device_malloc((void**)&attn_part_, part * 4));
   UAII_HIP(hipStreamSynchronize(stream_));
   max_ctx_ = max_seq;
   return Error::success();
@@ -887,14 +899,14 @@ Error DecoderProgram::arm_sampler(const SamplerParams& prm, const float* r, int6
   if (!samp_ws_) {
     const size_t b = sample_workspace_bytes(spec_.vocab);
     UAII_TRY(charge(used_static_, b));
-    UAII_HIP(hipMalloc(&samp_ws_, b));
+    UAII_HIP(device_malloc((void**)&samp_ws_, b));
     allocs_.push_back(samp_ws_);
   }
   if (n > samp_r_cap_) {
     if (samp_r_) (void)hipFree(samp_r_);
     samp_r_ = nullptr;
     samp_r_cap_ = 0;
-    UAII_HIP(hipMalloc((void**)&samp_r_, sizeof(float) * (size_t)n));
+    UAII_HIP(device_malloc((void**)&samp_r_, sizeof(float) * (size_t)n));
     samp_r_cap_ = n;
     // the graph holds the old buffer's address
     if (graph_[2]) (void)hipGraphExecDestroy(graph_[2]);

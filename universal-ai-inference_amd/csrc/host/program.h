@@ -149,6 +149,7 @@ class DecoderProgram {
   Error collect_timings();
   Error ensure_prefill_buffers(int64_t chunk);
   void release_prefill_buffers();  // the stream must be idle
+  hipError_t device_malloc(void** p, size_t bytes);
   Error prefill_rows(int64_t n);
   Error pf_gemm(const DeviceWeight* w[3], const int64_t cols0[3], int nw, const DeviceWeight* w2,
                 int epi, int64_t m, float* y, int64_t ldy, int store_split = 1);
