@@ -78,3 +78,17 @@ s.generate(prompt(40), 2)
 fake.fake_capacity(fake.fake_used() + 4096)
 s.generate_sampled(prompt(40), 4, uaii_amd.sample_params(temperature=0.8, top_k=5, seed=1))
 """)
+
+
+@pytest.mark.parametrize("f16", [False, True])
+def test_moe_without_ffn_norm_takes_steps(fake, tmp_path, f16):
+    """A MoE model without ffn_norm generates in token steps (the row routing needs the norm)."""
+    data = Path(synth.cached_model(MOE)).read_bytes()
+    assert data.count(b"ffn_norm.weight") == 2
+    path = tmp_path / "bare.gguf"
+    path.write_bytes(data.replace(b"ffn_norm.weight", b"ffn_none.weight"))
+    child(fake, path, """
+s = uaii_amd.Session(path, profile=True, kv_f16=%r)
+s.generate(prompt(40), 2)
+assert not rows(s) and not s.prefill_supported()
+""" % f16)

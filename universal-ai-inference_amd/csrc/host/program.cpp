@@ -370,7 +370,8 @@ Error DecoderProgram::build(const DecoderSpec& spec, const ProgramOptions& opts)
         ws.insert(ws.end(), {&L.gate_sh, &L.up_sh, &L.down_sh});
         if (L.inter_sh % 64) rows = false;
       }
-      if (!pf_router_supported(L.gate_inp.view.type)) rows = false;
+      // the row routing normalises its input; the token step's does either
+      if (!pf_router_supported(L.gate_inp.view.type) || !L.ffn_norm) rows = false;
     }
     if (ls.ffn != LayerSpec::kNone && ls.inter % 64) rows = false;
     for (const DeviceWeight* w : ws) {
