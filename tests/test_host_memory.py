@@ -92,3 +92,32 @@ s = uaii_amd.Session(path, profile=True, kv_f16=%r)
 s.generate(prompt(40), 2)
 assert not rows(s) and not s.prefill_supported()
 """ % f16)
+
+
+def test_prefill_budget(fake):
+    """The byte budget that lets an f16 session prefill 39 rows is no larger than what the
+    buffers have always come to: per row the stream, QKV, query, attention and hidden rows,
+    four splits of partials, hi + lo halves, one f32 a 32-block and a scale."""
+    d, q, kv, ffn, m, mpad = 512, 512, 128, 1024, 39, 64
+    budget = 4 * m * (d + (q + 2 * kv) + q + q + ffn) + 16 * m * (q + 2 * kv) + 4 * mpad * ffn + mpad * ffn // 8 + 4 * mpad
+    child(fake, synth.cached_model(DENSE), """
+def works(budget):
+    try:
+        s = uaii_amd.Session(path, budget_bytes=budget, kv_f16=True)
+        if ask: s.generate(prompt(40), 2)
+        s.close()
+        return True
+    except uaii_amd.UaiiError as e:
+        assert "memory budget exceeded" in str(e), e
+        return False
+least = []
+for ask in (False, True):
+    lo, hi = 1, 1 << 28
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        if works(mid): hi = mid
+        else: lo = mid
+    least.append(hi)
+print(least, least[1] - least[0])
+assert least[1] - least[0] <= %d
+""" % budget)

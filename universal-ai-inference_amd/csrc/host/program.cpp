@@ -447,7 +447,12 @@ Error DecoderProgram::ensure_prefill_buffers(int64_t chunk) {
   // (and, in short chunks, what feeds the down projection): 4 splits of a chunk's
   // rows, more in short chunks unless the session has a byte budget to keep
   pf_part_floats_ = 4 * chunk * std::max(d.dim, d.q_dim + 2 * d.kv_dim);
-  if (opts_.budget_bytes == 0)
+  // The sums' parts. Budgets were set when the sums took one f32 a 32-block: with one,
+  // what the parts take beyond that comes off the partials.
+  const size_t sum_bytes = pf_reads_ & PF_SUMS ? 64 * (size_t)((kmax + 255) / 256) * (size_t)mpad : 0;
+  if (opts_.budget_bytes != 0)
+    pf_part_floats_ -= std::clamp<int64_t>((int64_t)sum_bytes / 4 - kmax / 32 * mpad, 0, pf_part_floats_);
+  else
     pf_part_floats_ = std::max<int64_t>(pf_part_floats_, std::min<int64_t>(chunk, 64) * 16 * std::max(d.q_dim + 2 * d.kv_dim, 2 * inter));
   UAII_TRY(alloc(4 * (size_t)pf_part_floats_, (void**)&pf_part_));
   if (moe_) {
@@ -471,7 +476,7 @@ Error DecoderProgram::ensure_prefill_buffers(int64_t chunk) {
     UAII_TRY(alloc(2 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.hi));
     UAII_TRY(alloc(2 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.lo));
   }
-  if (pf_reads_ & PF_SUMS) UAII_TRY(alloc(64 * (size_t)((kmax + 255) / 256) * (size_t)mpad, (void**)&pf_act_.sxp));
+  if (pf_reads_ & PF_SUMS) UAII_TRY(alloc(sum_bytes, (void**)&pf_act_.sxp));
   if (pf_reads_ & PF_RAW) UAII_TRY(alloc(4 * (size_t)mpad * (size_t)kmax, (void**)&pf_act_.raw));
   UAII_TRY(alloc(4 * (size_t)mpad, (void**)&pf_act_.rs));
   pf_act_.mpad = mpad;
