@@ -377,8 +377,10 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn(PfAttnArgs a) {
     }
   };
   auto lds_barrier = []() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
   };
 
   auto compute = [&](int64_t kt, int buf) __attribute__((always_inline)) {
