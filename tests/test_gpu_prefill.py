@@ -173,13 +173,50 @@ def test_gemm_add_swiglu_wide_tile(hip, t):
     assert maxrel(dh.to_array(np.float32, m * rows).reshape(m, rows)[pick], want) < 1e-4
 
 
-def test_gemm_other_formats_run_row_by_row(hip):
-    """Formats outside the MFMA decoder go through the GEMV per row, same results."""
+def test_gemm_q5_k(hip):
+    """Five rows of a format that prefill() itself does not take."""
     t, rows, cols, m = uaii_amd.Q5_K, 200, 512, 5
     p = packed(t, rows, cols, 23)
     x = synth.normals(76, m, 0, m * cols, 1.0).reshape(m, cols)
     got = run_gemm(hip, DeviceWeight(t, p, rows, cols), x, rows)
     assert maxrel(got, oracle.quant_gemm(t, x, p, rows, nthreads=0)) < 1e-4
+
+
+@pytest.mark.parametrize("t,cols", [(uaii_amd.Q4_1, 512), (uaii_amd.Q5_0, 512), (uaii_amd.Q5_1, 512),
+                                    (uaii_amd.Q2_K, 512), (uaii_amd.Q3_K, 512), (uaii_amd.F32, 512),
+                                    (uaii_amd.Q8_0, 96), (uaii_amd.F16, 96)],
+                         ids=lambda v: uaii_amd.TYPE_NAMES[v] if v < 96 else str(v))
+def test_gemm_other_formats_run_row_by_row(hip, t, cols):
+    """Formats outside the MFMA decoder, and rows that are no multiple of 64, go through
+    the GEMV per row: the bits of the one-row entry points, for every epilogue."""
+    rows, m = 200, 5
+    pg, pu = packed(t, rows, cols, 23), packed(t, rows, cols, 24)
+    wg, wu = DeviceWeight(t, pg, rows, cols), DeviceWeight(t, pu, rows, cols)
+    x = synth.normals(76, m, 0, m * cols, 1.0).reshape(m, cols)
+    y0 = synth.normals(76, m, 1, m * rows, 1.0).reshape(m, rows)
+    dx, dn = DeviceBuffer.from_array(x), DeviceBuffer.from_array(1.0 + synth.normals(77, 1, 0, cols, 0.1))
+    at = lambda b, n: uaii_amd.C.c_void_p(b.ptr.value + 4 * n)
+    calls = {
+        "plain": (lambda y: hip.uaii_hip_gemm(wg.h, dx.ptr, m, y.ptr, None),
+                  lambda y, i: hip.uaii_hip_gemv(wg.h, at(dx, i * cols), at(y, i * rows), None)),
+        "rmsnorm": (lambda y: hip.uaii_hip_gemm_rmsnorm(wg.h, dx.ptr, m, dn.ptr, 1e-5, y.ptr, None),
+                    lambda y, i: hip.uaii_hip_gemv_rmsnorm(wg.h, at(dx, i * cols), dn.ptr, 1e-5, at(y, i * rows), None)),
+        "add": (lambda y: hip.uaii_hip_gemm_add(wg.h, dx.ptr, m, dn.ptr, 1e-5, y.ptr, None),
+                lambda y, i: hip.uaii_hip_gemv_add(wg.h, at(dx, i * cols), dn.ptr, 1e-5, at(y, i * rows), None)),
+        "swiglu": (lambda y: hip.uaii_hip_gemm_swiglu(wg.h, wu.h, dx.ptr, m, dn.ptr, 1e-5, y.ptr, None),
+                   lambda y, i: hip.uaii_hip_gemv_swiglu(wg.h, wu.h, at(dx, i * cols), dn.ptr, 1e-5, at(y, i * rows), None)),
+    }
+    for op, (gemm, gemv) in calls.items():
+        dy, dz = DeviceBuffer.from_array(y0), DeviceBuffer.from_array(y0)
+        check_hip(gemm(dy), op)
+        for i in range(m):
+            check_hip(gemv(dz, i), op)
+        check_hip(hip.uaii_hip_synchronize())
+        got, want = dy.to_array(np.float32, m * rows), dz.to_array(np.float32, m * rows)
+        assert np.array_equal(got, want), op
+        if op == "plain":
+            exact = x.astype(np.float64) @ oracle.dequant(t, pg, rows, cols).astype(np.float64).T
+            assert maxrel(got.reshape(m, rows), exact) < 1e-4
 
 
 @pytest.mark.parametrize("heads", [(8, 8, 64), (32, 8, 128), (16, 2, 64), (12, 4, 64), (6, 2, 128)],
