@@ -88,6 +88,17 @@ def test_row_gemm_large(hip, t, m, rows, cols, op):
     check(hip, op, t, m, rows, cols)
 
 
+# long rows: 16-, 32- and 64-row blocks on both sides of the lines in blocks times K, the
+# 32-row ones with 32 rows and with a ragged 64, and K splits of unequal shares
+@pytest.mark.parametrize("t", TYPES, ids=lambda t: uaii_amd.TYPE_NAMES[t])
+@pytest.mark.parametrize("m,rows,cols,op", [(100, 1000, 8192, "plain"), (100, 1030, 8192, "add"),
+                                            (17, 4100, 8192, "plain"), (65, 1000, 14336, "rmsnorm"),
+                                            (100, 700, 14336, "swiglu"), (300, 500, 14336, "add"),
+                                            (300, 1200, 512, "swiglu"), (500, 1408, 512, "swiglu")])
+def test_row_gemm_row_tiles(hip, t, m, rows, cols, op):
+    check(hip, op, t, m, rows, cols)
+
+
 def test_row_gemm_unaligned_output(hip):
     """y on a 4-byte boundary and an odd row count: the fold's one-column form."""
     t, m, rows, cols = uaii_amd.Q4_0, 5, 333, 2048

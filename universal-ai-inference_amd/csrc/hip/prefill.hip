@@ -275,8 +275,8 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn(PfAttnArgs a) {
   const int64_t nkeys = a.p0 + qend;  // keys the block needs (causal)
 
   // q * scale * 2^e as f16 hi + lo per query subtile u: lane (query col, group g)
-  // holds hd 32c + 8g .. +7 of chunk c; the matrix cores flush f16 subnormals,
-  // so each query row is scaled to put its largest element in [2^14, 2^15)
+  // holds hd 32c + 8g .. +7 of chunk c. Each query row is scaled to put its largest
+  // element in [2^14, 2^15): below 2^-14 f16 loses significant bits
   const float scale = 1.0f / sqrtf((float)HD);
   h8_t qhi[PA_QW][NC], qlo[PA_QW][NC];
   float qrs[PA_QW];
@@ -347,9 +347,9 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn(PfAttnArgs a) {
   const __half* kbase = reinterpret_cast<const __half*>(a.kcache) + (int64_t)kvh * a.max_seq * HD;
   const __half* vbase = reinterpret_cast<const __half*>(a.vcache) + (int64_t)kvh * a.max_seq * HD;
 
-  // tile staging: K pieces (key, 8 dims) and V pairs (keys 2k, 2k + 1, 8 dims);
-  // keys past nkeys read as zeros. Offsets inside a tile are 32-bit and fixed
-  // per thread; only the last tile checks them against nkeys.
+  // tile staging: pieces of 8 dims of a key, K and V alike; keys past nkeys read as
+  // zeros. Offsets inside a tile are 32-bit and fixed per thread; only the last tile
+  // checks them against nkeys.
   uint4 kreg[PIECES], vreg[PIECES];
   auto load_tile = [&](int64_t kt) __attribute__((always_inline)) {
     const __half* kt_base = reinterpret_cast<const __half*>(uniform_ptr(kbase + kt * HD));

@@ -33,10 +33,11 @@
 // Q6_K 120, 20.
 //
 // Block: 4 waves side by side along N, 16 MT rows x 64 NT columns. K runs in
-// stages of 64 (two 32-blocks), two LDS buffers in turn: everything a stage needs
-// travels global -> LDS (global_load_lds_dwordx4) while the stage before it is
-// computed, the block's A rows and each wave's own weight rows, so no registers hold
-// data in transit (held there, they spilled beside the accumulators). Lane group
+// stages of 64 (two 32-blocks) through two LDS buffers in turn, four in blocks of up to
+// 32 rows (see buffers): everything a stage needs travels global -> LDS
+// (global_load_lds_dwordx4) while the stages before it are computed, the block's A rows
+// and each wave's own weight rows, so no registers hold data in transit (held there,
+// they spilled beside the accumulators). Lane group
 // g = lane / 16 takes word g (4 bytes) of each 16-byte chunk of its row; with
 // 32-value blocks of two such halves that makes its eight k of a block the quads
 // 4 g .. and 16 + 4 g .., the order in which k_pf_prep stores A (see PfAct), for
@@ -44,8 +45,8 @@
 //
 // Scales. Q4_0 and Q8_0 blocks each have an f16 scale of their own, applied to the
 // block's f32 product. In Q4_K and Q5_K the 6-bit sub-block scale folds into the
-// integer: sc q <= 63 * 31 < 2048 is exact in f16 (one packed FMA from the
-// (1024 + q) form that the decode gives anyway), so the super-block's 256 k
+// integer: sc q <= 63 * 31 < 2048 is exact in f16 (one packed FMA from the (64 + q)
+// form that the decode gives anyway), so the super-block's 256 k
 // accumulate in the matrix core and only d is applied to the sum. Their minimums
 // are one more matrix op per super-block: the eight sub-block sums of A, each as
 // three f16 parts (all of its 24 bits), times the eight 6-bit minimums, then dmin.
@@ -799,14 +800,26 @@ int64_t col_tiles(const PfGemmArgs& a) {
 // for 64-row groups).
 int row_tiles(const PfGemmArgs& a) {
   if (a.gtab) return 4;
-  // Few blocks leave the chip to the latency of each one, which grows with its rows:
-  // microseconds at 16, 32, 64 rows a block, Q8_0 (blocks at 16 rows): 128 x 512 x 512
-  // (16) 13.4, 17.0, 23.5; 256 x 1408 x 512 SwiGLU (176) 15.0, 19.4, 23.1;
-  // 60 x 2048 x 2048 (32) 17.3, 20.6, 26.5; 100 x 4096 x 4096 (128) 37.9, 33.2, 34.5;
-  // 500 x 2048 x 2048 (256) 37.0, 34.0, 35.8; 250 x 8192 x 2048 SwiGLU (1024) 109, 81, 61
-  const int64_t b1 = col_tiles(a) * (a.mpad / 16);
-  if (a.mpad == 16 || b1 <= 64 || (a.K <= 1536 && b1 <= 192)) return 1;
-  return a.mpad == 32 || b1 <= 384 ? 2 : 4;
+  // Few blocks leave the chip to the latency of each one, which grows with its rows; but
+  // blocks of fewer rows read the weights more often, and leave less of the chip to split
+  // K over. So the line is one of blocks and of the K that they go through (b1, blocks at
+  // 16 rows, times K). Microseconds at 16, 32, 64 rows a block, whole calls:
+  //                        b1  b1 K / 2^18   Q8_0          Q4_K          Q6_K
+  //   100 x 1536 x 512     48  0.1          14  17  22    14  17  22    15  18  23
+  //   300 x 1408 x 512 +  220  0.4          15  20  24    16  20  24    18  21  25
+  //   500 x 1408 x 512 +  352  0.7          24  19  26    20  20  27    30  22  27
+  //   200 x 2048 x 2048   128  1            25  26  32    28  28  32    32  29  33
+  //   100 x 4096 x 4096   128  2            34  30  32    40  33  32    48  36  35
+  //   100 x 2048 x 8192    64  2            36  33  36    42  35  35    50  38  38
+  //   60 x 4096 x 14336    64  3.5          50  43  46    61  47  45    74  51  53
+  //   300 x 4096 x 4096   320  5            94  66  51    78  75  49   150  84  57
+  //   300 x 4096 x 14336  320  18          297 203 118   247 234 112   477 267 134
+  // (+ SwiGLU.) Q4_0 and Q5_K fall as Q8_0 and Q4_K do. F16's column tiles are half as
+  // wide: 100 x 4096 x 4096 74, 69, 60; 300 x 4096 x 14336 581, 818, 654.
+  // Q6_K, with half as many matrix ops again to a block, leaves 16 rows at half the line.
+  const int64_t b1 = col_tiles(a) * (a.mpad / 16), w = b1 * a.K;
+  if (a.mpad == 16 || (b1 <= 256 && w <= (1 << (a.seg[0].w.type == T_Q6_K ? 17 : 18)))) return 1;
+  return a.mpad == 32 || (b1 <= 384 && w <= (1 << 19)) ? 2 : 4;
 }
 
 // Wave groups per block: two where the grid has no more blocks than the chip has CUs.
