@@ -61,6 +61,17 @@ namespace {
 
 constexpr int GW = 4;  // waves side by side along N
 
+// Q8_0 with the K sums' rounding error carried along (PfGemmArgs::carry): the prompt rows
+// of sessions that ran them one token a step. Plain, the sums of 256 k were added one
+// after another, 16 to 56 of them, and the error grew past the step kernel's 1.09e-7 ..
+// 1.18e-7 of the result (1000 rows: 1.19e-7 at 14336 x 4096, 1.38e-7 at 4096 x 14336).
+// The carry takes the registers of half the columns, so its waves are 32 wide.
+// Carried: 0.93e-7 .. 1.10e-7 at every size, below the step kernel's there; 1000 rows
+// 303 -> 324 us at 14336 x 4096, 317 -> 334 at 4096 x 14336, 100 -> 103 at 4096 x 4096.
+constexpr int Q8_0_CARRY = 256 + T_Q8_0;
+template <int FMT>
+__device__ constexpr bool is_q8() { return FMT == T_Q8_0 || FMT == Q8_0_CARRY; }
+
 // Ties what computes v (or is computed from it) to this place: instruction selection
 // orders a block's pure arithmetic as it likes, and left to itself decodes several
 // subtiles ahead or leaves sums waiting, until registers spill (Q4_K, MT = 4: 168).
@@ -93,9 +104,9 @@ __device__ inline T ldg(gptr p, uint32_t o) {
 // same 32 bytes) and a dword of scales (Q4_0, Q8_0). Per two stages: Q6_K's high bits
 // of the half. Per four: a super-block's scales (16 bytes, and Q5_K's high bits).
 template <int FMT>
-constexpr int payload() { return FMT == T_F16 ? 128 : FMT == T_Q8_0 ? 64 : 32; }
+constexpr int payload() { return FMT == T_F16 ? 128 : is_q8<FMT>() ? 64 : 32; }
 template <int FMT>
-constexpr bool has_dword() { return FMT == T_Q4_0 || FMT == T_Q8_0; }
+constexpr bool has_dword() { return FMT == T_Q4_0 || is_q8<FMT>(); }
 
 // A super-block's scales of the lane's column, decoded from its 16 bytes.
 template <int FMT> struct Unit {};
@@ -136,7 +147,7 @@ __device__ inline void decode_block(const Words<FMT>& r, const Unit<FMT>& u, int
     const h2_t c = h2_of(-1032.0f), s = h2_of(0.0625f), e = h2_of(-72.0f);
     b = cat8(as_h2(and_or(w, kLo, 0x64006400u)) + c, as_h2(and_or(w8, kLo, 0x64006400u)) + c,
              pk_fma(as_h2(and_or(w, kHi, 0x64006400u)), s, e), pk_fma(as_h2(and_or(w8, kHi, 0x64006400u)), s, e));
-  } else if constexpr (FMT == T_Q8_0) {
+  } else if constexpr (is_q8<FMT>()) {
     const uint32_t v0 = r.w[0] ^ 0x80808080u, v1 = r.w[1] ^ 0x80808080u;
     const h2_t c = h2_of(-1152.0f);
     b = cat8(as_h2(byte_pair(v0)) + c, as_h2(byte_pair(v0 >> 8)) + c, as_h2(byte_pair(v1)) + c,
@@ -208,7 +219,7 @@ __device__ inline float block_scale(const Words<FMT>& r, int t) {
 // Column subtiles per wave. F16's 128 bytes per row and stage leave LDS for two
 // blocks per CU only with two (it has no decode to pay for, so its LDS reads may).
 template <int FMT>
-constexpr int nt_of() { return FMT == T_F16 ? 2 : 4; }
+constexpr int nt_of() { return FMT == T_F16 || FMT == Q8_0_CARRY ? 2 : 4; }
 
 // LDS: A stages [NB][block 2][hi/lo 2][BM rows][64 B], then per wave the payload
 // stages [NB][rows][payload], and for the formats that have them the dwords
@@ -254,6 +265,7 @@ template <int FMT, int EPI, int MT, int KH>
 __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
   constexpr int NT = nt_of<FMT>();
   constexpr bool F32 = FMT == T_F16;          // f32 operands
+  constexpr bool CARRY = F32 || FMT == Q8_0_CARRY;
   constexpr bool BLOCK_SCALE = !is_k<FMT>() && !F32;  // f32 sums per 32-block
   constexpr bool TWO = FMT != T_Q4_0 && !F32;  // sums per 256 k, then over K
   using L = Lds<FMT, MT>;
@@ -412,11 +424,15 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
   };
 
   const f4_t zero = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  f4_t acc[MT][NT], part[MT][NT];  // F32: part is what acc lost to rounding
+  f4_t acc[MT][NT], part[MT][NT];
+  f4_t lost[CARRY ? MT : 1][NT];  // what acc lost to rounding
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = part[i][j] = zero;
+    for (int j = 0; j < NT; ++j) {
+      acc[i][j] = part[i][j] = zero;
+      if constexpr (CARRY) lost[i][j] = zero;
+    }
 
   Unit<FMT> unit[NT];
 
@@ -444,7 +460,7 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
     const uint32_t o = buf * L::W + 16 * j * payload<FMT>();
     if constexpr (FMT == T_Q4_0) {
       r.w[0] = lw(o + poff[t]);
-    } else if constexpr (FMT == T_Q8_0) {
+    } else if constexpr (is_q8<FMT>()) {
       r.w[0] = lw(o + poff[2 * t]);
       r.w[1] = lw(o + poff[2 * t + 1]);
     } else if constexpr (FMT == T_F16) {
@@ -618,10 +634,10 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
           const f4_t add = (s8[0][i] + s8[1][i]) + (s8[2][i] + s8[3][i]), to = acc[i][j] + add;
-          part[i][j] += add - (to - acc[i][j]);
+          lost[i][j] += add - (to - acc[i][j]);
           acc[i][j] = to;
           pin(acc[i][j]);
-          pin(part[i][j]);
+          pin(lost[i][j]);
         }
       } else {
         constexpr bool first = h == 0 && t == 0;  // of the unit
@@ -671,6 +687,11 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
         for (int j = 0; j < NT; ++j) {
           if constexpr (is_k<FMT>()) {
             acc[i][j] += unit[j].d * part[i][j];
+          } else if constexpr (CARRY) {
+            const f4_t to = acc[i][j] + part[i][j];
+            lost[i][j] += part[i][j] - (to - acc[i][j]);
+            acc[i][j] = to;
+            pin(lost[i][j]);
           } else {
             acc[i][j] += part[i][j];
           }
@@ -679,14 +700,14 @@ __global__ void __launch_bounds__(GW * 64 * KH, 2 / KH) k_pf_mm(PfGemmArgs a) {
     }
   }
 
-  if constexpr (F32) {
+  if constexpr (CARRY) {
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r)  // an infinite sum has nothing beside it
-          if (isfinite(acc[i][j][r])) acc[i][j][r] += part[i][j][r];
+          if (isfinite(acc[i][j][r])) acc[i][j][r] += lost[i][j][r];
   }
 
   if constexpr (KH == 2) {
@@ -788,9 +809,16 @@ hipError_t go(PfGemmArgs a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The kernel's format.
+int kernel_fmt(const PfGemmArgs& a) {
+  const int type = a.seg[0].w.type;
+  return a.carry && type == T_Q8_0 ? Q8_0_CARRY : type;
+}
+
 // Column tiles of a launch.
 int64_t col_tiles(const PfGemmArgs& a) {
-  const int per = GW * 16 * (a.seg[0].w.type == T_F16 ? 2 : 4) / (a.epi == EPI_SWIGLU ? 2 : 1);
+  const int fmt = kernel_fmt(a);
+  const int per = GW * 16 * (fmt == T_F16 || fmt == Q8_0_CARRY ? 2 : 4) / (a.epi == EPI_SWIGLU ? 2 : 1);
   int64_t n = 0;
   for (int k = 0; k < a.nseg; ++k) n += (a.seg[k].rows + per - 1) / per;
   return n;
@@ -935,9 +963,10 @@ hipError_t launch_pf_gemm(PfGemmArgs a, hipStream_t s) {
     if (a.epi == EPI_SWIGLU && (sg.w2.type != type || sg.w2.cols != a.K || sg.rows > sg.w2.rows))
       return hipErrorInvalidValue;
   }
-  switch (type) {
+  switch (kernel_fmt(a)) {
     case T_Q4_0: return go_epi<T_Q4_0>(a, s);
     case T_Q8_0: return go_epi<T_Q8_0>(a, s);
+    case Q8_0_CARRY: return go_epi<Q8_0_CARRY>(a, s);
     case T_F16: return go_epi<T_F16>(a, s);
     case T_Q4_K: return go_epi<T_Q4_K>(a, s);
     case T_Q5_K: return go_epi<T_Q5_K>(a, s);

@@ -296,6 +296,9 @@ struct PfGemmArgs {
   // (MoE experts gather their tokens); rows are those of ahi/alo/sxp/rs
   const int32_t* arow;
   int64_t act_ld;  // the activations' padded row count; 0: mpad
+  // Q8_0: the rows stand for token steps, whose sums over K round less (prefill_gemm.hip);
+  // the other formats' sums do not
+  int carry;
   // optional expert grouping (MoE): grid row y computes output rows
   // [gtab[3y + 1], gtab[3y + 2]) against expert gtab[3y] of the weight stacks,
   // whose rows e * seg.rows .. (e + 1) * seg.rows - 1 are that expert's;

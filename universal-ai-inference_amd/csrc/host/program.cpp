@@ -497,6 +497,7 @@ Error DecoderProgram::pf_gemm(const DeviceWeight* w[3], const int64_t cols0[3], 
     a.M = m;
     a.K = w[i]->view.cols;
     a.mpad = pf_act_.mpad;
+    a.carry = !pf_ok_;  // such a session's prompts were token steps
     pf_take(pf_act_, w[i]->view.type, &a);
     a.y = y;
     a.ldy = ldy;
@@ -549,6 +550,7 @@ int DecoderProgram::pf_store_split(const DeviceWeight* w[3], int nw, int64_t m, 
     a.M = m;
     a.K = w[i]->view.cols;
     a.mpad = pf_act_.mpad;
+    a.carry = !pf_ok_;
     int j = i;
     while (j < nw && w[j]->view.type == w[i]->view.type) {
       PfSeg& sg = a.seg[a.nseg++];
@@ -640,6 +642,7 @@ Error DecoderProgram::prefill_moe(const Layer& L, const LayerSpec& ls, int64_t m
     g.seg[0].w = w.view;
     pf_take(pf_act_, w.view.type, &g);
     g.act_ld = pf_act_.mpad;
+    g.carry = !pf_ok_;
     g.gtab = pf_moe_tab_ + 3 * t0;
     g.ntab = nt;
     g.ngroups = E;
