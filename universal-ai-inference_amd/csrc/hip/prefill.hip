@@ -814,7 +814,9 @@ hipError_t launch_pf_prep(float* x, int64_t ldx, int64_t M, const float* norm_w,
     UAII_LAUNCH(kernel, dim3((unsigned)act.mpad), dim3(threads), lds, s, x, ldx, M, norm_w, eps, act, part, nsplit);
     return hipGetLastError();
   };
-  // up to a block per two CUs the row's own latency is the launch's
+  // Up to a block per two CUs the row's own latency is the launch's: whole products of 9
+  // to 100 rows take 3-4 % less with 1024 threads (six formats, K of 1408 to 14336), of
+  // 300 and 500 rows 0.5 %, at K = 512 up to 3 % more.
   return act.mpad <= 128 && act.K >= 1024 ? go(&k_pf_prep<1024>, 1024) : go(&k_pf_prep<256>, 256);
 }
 
