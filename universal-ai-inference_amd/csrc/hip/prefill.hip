@@ -240,7 +240,7 @@ __device__ inline int pf_attn_tile(int xi, int nx, int band) {
 // V was stored transposed, 4 bytes a lane with rows 288 words apart: 8 lanes to a bank
 // on every store, as much LDS time as all fragment reads together, and 16 vector
 // operations a piece to pair the keys. Stored plain and read by ds_read_b64_tr_b16
-// (two conflict-free reads a fragment, as before), with the probabilities' hi and lo
+// (two reads a fragment, as before), with the probabilities' hi and lo
 // halves one fused operation each: 1024 queries at 1024, 32/8 heads of 128,
 // 139 -> 80 us between calls from the host, 138 -> 66 back to back with the band order
 // below (25.8 GFLOP: 187 -> 391 TFLOP/s); 512 queries at 4096 210 -> 125 us, where one
